@@ -47,8 +47,8 @@ thread_local bool lastPacked = false; // operands went through gemm_pack_rows
 
 // ---------------------------------------------------------------------------
 // C[M,N] = alpha * A[M,K] * B[K,N] + beta * C with C row-major (ldc) on the
-// matrix cores, float32 (v_mfma_f32_32x32x2_f32) or float64
-// (v_mfma_f64_16x16x4_f64), accumulating in the operand type.  Each input
+// float64 matrix cores (v_mfma_f64_16x16x4_f64); float32 products are
+// sgemm_parts (SgemmParts.h), which takes the same arguments.  Each input
 // operand may be stored with either of its two dimensions contiguous:
 //   A_KC: A(m,k) = A[m * lda + k]   (row-major A)   else A[k * lda + m]
 //   B_NC: B(k,n) = B[k * ldb + n]   (row-major B)   else B[n * ldb + k]
@@ -56,13 +56,11 @@ thread_local bool lastPacked = false; // operands went through gemm_pack_rows
 // handled by the host as C^T = B^T A^T.
 //
 // 256 threads = 4 waves in a 2 x 2 grid; each wave owns TM x TN MFMA tiles of
-// edge TILE (32 for float32, 16 for float64), so the block tile is
-// (2 TM TILE) x (2 TN TILE).  K advances in slabs of BK elements (16, or 32
-// for the large float32 tile).
+// edge 16, so the block tile is (32 TM) x (32 TN).  K advances in slabs of 16.
 //
 // LDS holds both operands K-major ([k][m] and [k][n], rows padded so that the
 // rows one MFMA operand fetch touches fall on different banks): lane l needs
-// element (l % TILE) of row (k + l / TILE), a conflict-free ds_read.  Global
+// element (l % 16) of row (k + l / 16), a conflict-free ds_read.  Global
 // fetches are 128-bit along the operand's contiguous dimension: an operand
 // contiguous in m / n is written to LDS as one 128-bit word, one contiguous
 // in k is scattered over LDS rows.  Two LDS stages: the next K slab is
@@ -72,8 +70,7 @@ thread_local bool lastPacked = false; // operands went through gemm_pack_rows
 // the slab loop).
 //
 // MFMA operand layouts (64 lanes):
-//   f32 32x32x2: A[l % 32][l / 32], B[l / 32][l % 32],
-//                D reg r = D[8*(r/4) + 4*(l/32) + r%4][l % 32]   (16 regs)
+//   f32 32x32 (any K): D reg r = D[8*(r/4) + 4*(l/32) + r%4][l % 32]  (16 regs)
 //   f64 16x16x4: A[l % 16][l / 16], B[l / 16][l % 16],
 //                D reg r = D[4*r + l/16][l % 16]                  (4 regs)
 //
@@ -83,16 +80,8 @@ thread_local bool lastPacked = false; // operands went through gemm_pack_rows
 // dimension multiples of the vector.
 template <typename T> struct Mfma;
 template <> struct Mfma<float> {
-  typedef floatx4 Vec;   // 128-bit global access
-  typedef floatx16 Acc;  // one MFMA tile per lane
-  static constexpr int TILE = 32, KSTEP = 2, BK = 16, VEC = 4, NACC = 16,
-                       PAD = 4;
-  // LDS reads after the compiler has paired them: one ds_read2_b32 for two
-  // fragments a tile apart.
-  static constexpr int fragmentReads(int fragments) { return fragments / 2; }
-  __device__ static __forceinline__ Acc mma(float a, float b, Acc c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-  }
+  typedef floatx4 Vec; // 128-bit global access
+  static constexpr int BK = 16, VEC = 4;
   __device__ static __forceinline__ int accRow(int r, int lane) {
     return 8 * (r / 4) + 4 * (lane / 32) + r % 4;
   }
@@ -121,8 +110,10 @@ template <> struct Mfma<double> {
 // lies outside it (words are whole: the host checks that the extents along
 // the contiguous dimension are multiples of the word) is read from the
 // operand's first word instead and replaced by zeros.
-template <typename T, int X, int BK, bool K_CONTIG, bool GUARD> struct SlabFetch {
+template <int X, bool K_CONTIG, bool GUARD> struct SlabFetch {
+  typedef double T;
   typedef Mfma<T> M;
+  static constexpr int BK = M::BK;
   typedef typename M::Vec Vec;
   static constexpr int NV = X * BK / (M::VEC * 256);
   static constexpr int X_STEP = 256 * M::VEC / BK; // K_CONTIG: x rows per pass
@@ -193,8 +184,8 @@ template <int MASK> __device__ __forceinline__ void sched_groups(int n) {
   if (n > 3) __builtin_amdgcn_sched_group_barrier(MASK, 1, 0);
 }
 
-// float64 tiles need under 256 registers a lane: two blocks share a CU and
-// fill each other's stalls.  float32 256 x 256 tiles take a CU each.
+// Under 256 registers a lane: two blocks share a CU and fill each other's
+// stalls.
 //
 // Split K (sliceK > 0): grid.z slices of sliceK elements of K (a multiple of
 // BK) each; slice z leaves its unscaled partial product in the workspace,
@@ -229,13 +220,14 @@ __host__ __device__ inline int64_t evenSharesStart(int64_t g, int64_t units,
 // GUARD: 0 whole tiles; 1 loads and stores guarded (operands and C of any
 // extent); 2 stores alone guarded (operands padded with zeros to whole tiles
 // and slabs, C of any extent).
-template <typename T, int BK, int TM, int TN, bool A_KC, bool B_NC, int GUARD = 0>
-__global__ __launch_bounds__(256, sizeof(T) == 8 ? 2 : 1) void
-gemm_mfma(const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C,
-          int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, T alpha,
-          T beta, int sliceK, T *__restrict__ W, int64_t ldw, EvenShares even) {
+template <int TM, int TN, bool A_KC, bool B_NC, int GUARD>
+__global__ __launch_bounds__(256, 2) void
+dgemm_mfma(const double *__restrict__ A, const double *__restrict__ B, double *__restrict__ C,
+           int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, double alpha,
+           double beta, int sliceK, double *__restrict__ W, int64_t ldw, EvenShares even) {
+  typedef double T;
   typedef Mfma<T> MF;
-  constexpr int TILE = MF::TILE;
+  constexpr int TILE = MF::TILE, BK = MF::BK;
   constexpr int BM = 2 * TM * TILE, BN = 2 * TN * TILE;
   __shared__ __attribute__((aligned(16))) T As[2][BK][BM + MF::PAD];
   __shared__ __attribute__((aligned(16))) T Bs[2][BK][BN + MF::PAD];
@@ -283,8 +275,8 @@ gemm_mfma(const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C,
   unit += slab1 - slab0;
   const bool piece = even.slabs > 0 && !(slab0 == 0 && slab1 == even.slabs);
 
-  SlabFetch<T, BM, BK, A_KC, GUARD == 1> fa;
-  SlabFetch<T, BN, BK, !B_NC, GUARD == 1> fb;
+  SlabFetch<BM, A_KC, GUARD == 1> fa;
+  SlabFetch<BN, !B_NC, GUARD == 1> fb;
   fa.init(A, lda, bm, tid, M, K);
   fb.init(B, ldb, bn, tid, N, K);
 
@@ -431,8 +423,31 @@ gemm_mfma(const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C,
   } // segments
 }
 
+} // namespace
+
+#include "SgemmParts.h"
+
+namespace {
+
+// The tile kernel of a type and block tile, and its threads: float32 products
+// in bf16 parts (both tiles guard themselves), float64 ones on the float64
+// matrix cores.
+template <typename T, int TILE, bool A_KC, bool B_NC, int GUARD> struct TileKernel;
+template <bool A_KC, bool B_NC, int GUARD> struct TileKernel<float, 256, A_KC, B_NC, GUARD> {
+  static constexpr int THREADS = 512;
+  static constexpr auto kernel = sgemm_parts<256, 256, 2, 4, A_KC, B_NC>;
+};
+template <bool A_KC, bool B_NC, int GUARD> struct TileKernel<float, 128, A_KC, B_NC, GUARD> {
+  static constexpr int THREADS = 256;
+  static constexpr auto kernel = sgemm_parts<128, 128, 2, 2, A_KC, B_NC>;
+};
+template <bool A_KC, bool B_NC, int GUARD> struct TileKernel<double, 128, A_KC, B_NC, GUARD> {
+  static constexpr int THREADS = 256;
+  static constexpr auto kernel = dgemm_mfma<4, 4, A_KC, B_NC, GUARD>;
+};
+
 // ---------------------------------------------------------------------------
-// The tiles that gemm_mfma's even shares cut into pieces: C[tile] = alpha *
+// The tiles that the even shares cut into pieces: C[tile] = alpha *
 // (piece + piece + ...) + beta * C[tile], pieces in K order (the order of the
 // blocks that computed them: a fixed order).  One block per tile row-chunk:
 // grid (tiles, BM * BN / (256 * VEC * ROWS))...  A thread owns one 128-bit
@@ -1812,19 +1827,17 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       // (4000^3: 3968 x 3968 x 4000 on the matrix cores, 26 -> 65 TFLOP/s).
       // float32: 256 x 256 block tiles (one block per CU on a 4096^2
       // problem) when the shape allows and there are enough tiles to fill the
-      // 256 CUs, 128 x 128 otherwise (measured within 3 % of each other; the
-      // larger tile halves the operand traffic).  float64: 128 x 128.  The
-      // large tile advances K in slabs of 2 BK where K allows (half the
-      // barriers; 144 against 142 TFLOP/s on 4096^3).
+      // 256 CUs, 128 x 128 otherwise (4096^3: 577 against 704 us; the larger
+      // tile halves the operand traffic and the splitting into parts).
+      // float64: 128 x 128.
       const int64_t Mt = Mz - Mz % 128, Nt = Nz - Nz % 128, Kt = K - K % BK;
       // Where whole tiles would leave CUs idle (too few of them, or a last
       // round that is mostly empty) and K is long enough, the blocks take
       // even shares of the K slabs of all tiles instead (planEvenShares).
       const bool bigFits = sizeof(T) == 4 && Mt % 256 == 0 && Nt % 256 == 0;
       const int64_t bigTiles = (Mt / 256) * (Nt / 256);
-      const int bigSlab = Kt % (2 * BK) == 0 ? 2 * BK : BK;
       const int bigEven = bigFits && workspaceKind == WORKSPACE_HEAP
-                              ? planEvenShares(bigTiles, Kt / bigSlab, cus)
+                              ? planEvenShares(bigTiles, Kt / BK, cus)
                               : 0;
       // (from 64 large tiles on: below, the 128 x 128 tiles in slices or
       // shares are as fast or faster -- 1792^3 120 against 131 us, 1024 x
@@ -1888,17 +1901,15 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       // copies have to be won back from the guards on the loads alone).
       bool paddedBig = false;
       {
-        // float32: 256 x 256 tiles, K slabs of 32; float64: 128 x 128, slabs of 16
         constexpr int PT = sizeof(T) == 4 ? 256 : 128;
-        constexpr int PSLAB = sizeof(T) == 4 ? 2 * BK : BK;
         const int64_t padSlots = sizeof(T) == 4 ? cus : slots;
         const int64_t minTiles = sizeof(T) == 4 ? 3 * cus / 4 : cus;
         auto roundUp = [](int64_t v, int64_t to) { return (v + to - 1) / to * to; };
-        const int64_t Mp = roundUp(Mz, PT), Np = roundUp(Nz, PT), Kp = roundUp(K, PSLAB);
+        const int64_t Mp = roundUp(Mz, PT), Np = roundUp(Nz, PT), Kp = roundUp(K, BK);
         const bool fitsAsIs = Mz == Mp && Nz == Np && K % BK == 0 && !offWords(X, ldx, xC) &&
                               !offWords(Y, ldy, yC);
         const int64_t padTiles = (Mp / PT) * (Np / PT);
-        const int slabs = int(Kp / PSLAB);
+        const int slabs = int(Kp / BK);
         int evenBlocks = planEvenShares(padTiles, slabs, padSlots);
         if (!launched && canPack && !fitsAsIs && (!whole || packX || packY) && K >= 256 &&
             padTiles >= minTiles &&
@@ -1933,10 +1944,10 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
             if (evenBlocks)
               grid = dim3(unsigned(evenBlocks), 1, 1);
 #define NMHIP_GEMM_PADDED(XKC, YNC)                                            \
-  hipLaunchKernelGGL((gemm_mfma<T, PSLAB, 4, 4, XKC, YNC, 2>), grid,          \
-                     dim3(256), 0, stream, Xp, Yp, cData, int(Mz), int(Nz),    \
-                     int(Kp), xCp, yCp, ldz, alpha, beta, 0, W, int64_t(0),    \
-                     even)
+  hipLaunchKernelGGL((TileKernel<T, PT, XKC, YNC, 2>::kernel), grid,           \
+                     dim3(TileKernel<T, PT, XKC, YNC, 2>::THREADS), 0, stream, \
+                     Xp, Yp, cData, int(Mz), int(Nz), int(Kp), xCp, yCp, ldz,  \
+                     alpha, beta, 0, W, int64_t(0), even)
             if (xKc && yNc)
               NMHIP_GEMM_PADDED(true, true);
             else if (xKc)
@@ -2024,29 +2035,24 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
         dim3 grid(unsigned(tilesN), unsigned(tilesM), unsigned(plan.slices));
         if (evenBlocks)
           grid = dim3(unsigned(evenBlocks), 1, 1);
-#define NMHIP_GEMM_RAGGED(TM, TN, XKC, YNC)                                    \
-  hipLaunchKernelGGL((gemm_mfma<T, BK, TM, TN, XKC, YNC, 1>), grid,            \
-                     dim3(256), 0, stream, X, Y, cData, int(Mz), int(Nz),      \
-                     int(K), ldxk, ldyk, ldz, alpha, beta, plan.sliceK, W, ldw,\
-                     even)
-#define NMHIP_GEMM_RAGGED_LAYOUTS(TM, TN)                                      \
-  do {                                                                         \
-    if (xKc && yNc)                                                            \
-      NMHIP_GEMM_RAGGED(TM, TN, true, true);                                   \
-    else if (xKc)                                                              \
-      NMHIP_GEMM_RAGGED(TM, TN, true, false);                                  \
-    else if (yNc)                                                              \
-      NMHIP_GEMM_RAGGED(TM, TN, false, true);                                  \
-    else                                                                       \
-      NMHIP_GEMM_RAGGED(TM, TN, false, false);                                 \
-  } while (0)
+#define NMHIP_GEMM_RAGGED(XKC, YNC)                                            \
+  hipLaunchKernelGGL((TileKernel<T, 128, XKC, YNC, 1>::kernel), grid,          \
+                     dim3(TileKernel<T, 128, XKC, YNC, 1>::THREADS), 0, stream,\
+                     X, Y, cData, int(Mz), int(Nz), int(K), ldxk, ldyk, ldz,   \
+                     alpha, beta, plan.sliceK, W, ldw, even)
+        if (xKc && yNc)
+          NMHIP_GEMM_RAGGED(true, true);
+        else if (xKc)
+          NMHIP_GEMM_RAGGED(true, false);
+        else if (yNc)
+          NMHIP_GEMM_RAGGED(false, true);
+        else
+          NMHIP_GEMM_RAGGED(false, false);
         if constexpr (sizeof(T) == 4) {
-          NMHIP_GEMM_RAGGED_LAYOUTS(2, 2);
           lastKernel = evenBlocks        ? "sgemm_mfma_128x128_ragged_even"
                        : plan.slices > 1 ? "sgemm_mfma_128x128_ragged_splitk"
                                          : "sgemm_mfma_128x128_ragged";
         } else {
-          NMHIP_GEMM_RAGGED_LAYOUTS(4, 4);
           lastKernel = evenBlocks        ? "dgemm_mfma_128x128_ragged_even"
                        : plan.slices > 1 ? "dgemm_mfma_128x128_ragged_splitk"
                                          : "dgemm_mfma_128x128_ragged";
@@ -2056,15 +2062,13 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
           evenFold(W, evenBlocks, slabs, tilesM, tilesN, 128, Mz, Nz, ldz, cData);
         else if (plan.slices > 1)
           fold(plan, W, Mz, Nz, ldw, ldz, cData);
-#undef NMHIP_GEMM_RAGGED_LAYOUTS
 #undef NMHIP_GEMM_RAGGED
         launched = true;
       } else if (unitOk && mostly && Mt > 0 && Nt > 0 && Kt > 0 &&
           ldx % VEC == 0 && ldy % VEC == 0 && ldx > 0 && ldy > 0 &&
           aligned16(X) && aligned16(Y) && M <= 0x7fffffff && N <= 0x7fffffff &&
           K <= 0x7fffffff && Mz <= 65535 * 32) {
-        const int slabK = big ? bigSlab : BK;
-        const int slabs = int(Kt / slabK);
+        const int slabs = int(Kt / BK);
         SplitPlan plan;
         bool slicesFill = false;
         if (!big)
@@ -2084,28 +2088,27 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
         dim3 grid(unsigned(Nt / BN), unsigned(Mt / BM), unsigned(plan.slices));
         if (evenBlocks)
           grid = dim3(unsigned(evenBlocks), 1, 1);
-#define NMHIP_GEMM_LAUNCH(SLAB, TM, TN, XKC, YNC)                              \
-  hipLaunchKernelGGL((gemm_mfma<T, SLAB, TM, TN, XKC, YNC>), grid, dim3(256),  \
-                     0, stream, X, Y, cData, int(Mt), int(Nt), int(Kt), ldx,   \
-                     ldy, ldz, alpha, beta, plan.sliceK, W, int64_t(Nt), even)
-#define NMHIP_GEMM_LAYOUTS(SLAB, TM, TN)                                       \
+#define NMHIP_GEMM_LAUNCH(TILE, XKC, YNC)                                      \
+  hipLaunchKernelGGL((TileKernel<T, TILE, XKC, YNC, 0>::kernel), grid,         \
+                     dim3(TileKernel<T, TILE, XKC, YNC, 0>::THREADS), 0,       \
+                     stream, X, Y, cData, int(Mt), int(Nt), int(Kt), ldx, ldy, \
+                     ldz, alpha, beta, plan.sliceK, W, int64_t(Nt), even)
+#define NMHIP_GEMM_LAYOUTS(TILE)                                               \
   do {                                                                         \
     if (xKc && yNc)                                                            \
-      NMHIP_GEMM_LAUNCH(SLAB, TM, TN, true, true);                             \
+      NMHIP_GEMM_LAUNCH(TILE, true, true);                                     \
     else if (xKc)                                                              \
-      NMHIP_GEMM_LAUNCH(SLAB, TM, TN, true, false);                            \
+      NMHIP_GEMM_LAUNCH(TILE, true, false);                                    \
     else if (yNc)                                                              \
-      NMHIP_GEMM_LAUNCH(SLAB, TM, TN, false, true);                            \
+      NMHIP_GEMM_LAUNCH(TILE, false, true);                                    \
     else                                                                       \
-      NMHIP_GEMM_LAUNCH(SLAB, TM, TN, false, false);                           \
+      NMHIP_GEMM_LAUNCH(TILE, false, false);                                   \
   } while (0)
         if constexpr (sizeof(T) == 4) {
-          if (big && bigSlab == 2 * BK)
-            NMHIP_GEMM_LAYOUTS(2 * BK, 4, 4);
-          else if (big)
-            NMHIP_GEMM_LAYOUTS(BK, 4, 4);
+          if (big)
+            NMHIP_GEMM_LAYOUTS(256);
           else
-            NMHIP_GEMM_LAYOUTS(BK, 2, 2);
+            NMHIP_GEMM_LAYOUTS(128);
           static const char *const names[2][4][2] = {
               {{"sgemm_mfma_128x128", "sgemm_mfma_128x128+edges"},
                {"sgemm_mfma_128x128_splitk", "sgemm_mfma_128x128_splitk+edges"},
@@ -2117,7 +2120,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
                {"", ""}}};
           lastKernel = names[big ? 1 : 0][evenBlocks ? 2 : plan.slices > 1 ? 1 : 0][whole ? 0 : 1];
         } else {
-          NMHIP_GEMM_LAYOUTS(BK, 4, 4);
+          NMHIP_GEMM_LAYOUTS(128);
           lastKernel = evenBlocks ? (whole ? "dgemm_mfma_128x128_even"
                                            : "dgemm_mfma_128x128_even+edges")
                        : plan.slices > 1
