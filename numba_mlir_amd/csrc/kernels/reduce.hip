@@ -451,72 +451,165 @@ reduceStrided(const IN *x, ACC *out, int64_t nKeep, int64_t nRed, int64_t sk,
     out[k * so] = acc;
 }
 
+// Fold of v[0 .. N) (N a power of two) in pairs, in place.
+template <int N, typename ACC, typename Op>
+__device__ __forceinline__ ACC foldInPairs(ACC (&v)[N], Op op) {
+#pragma unroll
+  for (int half = N / 2; half > 0; half /= 2)
+#pragma unroll
+    for (int u = 0; u < half; ++u)
+      v[u] = op(v[u], v[u + half]);
+  return v[0];
+}
+
 // Generic reduction over the slow axis of a matrix whose kept index has unit
-// stride (column sums of a row-major matrix, row sums of a column-major one):
-// out[chunk * nKeep + k] = fold_{r in chunk} op(x[r * ld + k]); with more than
-// one chunk the same kernel folds the partial results.
-// vec == 0: a block owns 256 consecutive kept indices, one a lane, and a
-// chunk of rowsPerChunk reduced indices, eight loads in flight per lane.
-// vec != 0 (the host has checked: x 16-byte aligned, ld and nKeep multiples
-// of the elements in a 128-bit word): a block owns a strip of 64 words (1 KiB
-// of every row), a word a lane; its four waves take interleaved rows of the
-// chunk, eight loads in flight per lane, and meet in LDS.
+// stride (column sums of a row-major matrix, row sums of a column-major one),
+// in chunks of rowsPerChunk reduced indices along grid.y.
+//
+// words != 0 (nKeep holds a 128-bit word or more): a lane reads 128-bit words,
+// eight in flight, on whatever element they begin -- the memory pipe takes
+// them at any element boundary, so rows of odd extents and leading dimensions
+// stream like aligned ones.  The word that would end beyond the row is read
+// further left, from the row's last whole word, and gives only its last
+// elements.  1 << (words - 1) lanes (at most a wave) lie side by side along a
+// row and own a strip of it; the rest of the block's 256 lanes take
+// interleaved rows of the chunk and meet in LDS, so narrow matrices fill the
+// waves too.  With tickets (several chunks) the block that draws the last
+// ticket of its strip folds the chunks in index order: one launch, where a
+// second one over the partial results cost 9 us and the gap before it.
+// Bound by memory: [5003, 3001] int32 column sums (60 MB) take 16.1 us, in two
+// launches of one element a lane 21.7.
+//
+// words == 0 (rows shorter than a word, or more strips than tickets): a block
+// owns 256 consecutive kept indices, one a lane, eight loads in flight;
+// several chunks leave their results at out[chunk * nKeep + k], and the same
+// kernel folds them.
 template <typename IN, typename ACC, typename Op>
 __device__ __forceinline__ void
 reduceColumns(const IN *__restrict__ x, ACC *__restrict__ out, int64_t nRed,
-              int64_t nKeep, int64_t ld, int64_t rowsPerChunk, int32_t vec, ACC init,
-              Op op) {
+              int64_t nKeep, int64_t ld, int64_t rowsPerChunk, int32_t words,
+              ACC *partial, uint32_t *tickets, ACC init, Op op) {
   int64_t r = int64_t(blockIdx.y) * rowsPerChunk;
   int64_t rEnd = r + rowsPerChunk;
   if (rEnd > nRed)
     rEnd = nRed;
-  if (vec) {
-    typedef typename WordOf<IN>::type Word;
+  if (words) {
     constexpr int N = WordOf<IN>::N;
-    constexpr int WAVES = 256 / NMK_WAVE;
+    typedef IN Word __attribute__((ext_vector_type(N), aligned(sizeof(IN))));
     constexpr int U = 8;
-    __shared__ ACC meet[WAVES][NMK_WAVE * N];
-    const int lane = threadIdx.x % NMK_WAVE;
-    const int wave = threadIdx.x / NMK_WAVE;
-    const int64_t k = (int64_t(blockIdx.x) * NMK_WAVE + lane) * N;
+    __shared__ ACC meet[256 * N];
+    __shared__ uint32_t isLast;
+    const int shift = words - 1, across = 1 << shift, down = 256 >> shift;
+    const int inStrip = threadIdx.x & (across - 1);
+    const int64_t strip0 = int64_t(blockIdx.x) * across * N;
+    const int64_t k = strip0 + int64_t(inStrip) * N;
+    const int64_t from = k + N <= nKeep ? k : nKeep - N; // where its word is read
     ACC a[N];
 #pragma unroll
     for (int q = 0; q < N; ++q)
       a[q] = init;
     if (k < nKeep) {
-      r += wave;
-      const IN *p = x + r * ld + k;
-      const int64_t step = WAVES * ld;
-      for (; r + WAVES * (U - 1) < rEnd; r += WAVES * U) {
+      r += threadIdx.x >> shift;
+      const IN *p = x + r * ld + from;
+      const int64_t step = down * ld;
+      for (; r + down * (U - 1) < rEnd; r += down * U) {
         Word v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
           v[u] = __builtin_nontemporal_load(reinterpret_cast<const Word *>(p + u * step));
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int q = 0; q < N; ++q) {
+          // (in pairs: the chain of sums is an eighth as long, and gathers less
+          // rounding)
+          ACC s[U];
 #pragma unroll
-          for (int q = 0; q < N; ++q)
-            a[q] = op(a[q], ACC(v[u][q]));
+          for (int u = 0; u < U; ++u)
+            s[u] = ACC(v[u][q]);
+          a[q] = op(a[q], foldInPairs<U>(s, op));
+        }
         p += U * step;
       }
-      for (; r < rEnd; r += WAVES) {
-        const Word v = __builtin_nontemporal_load(reinterpret_cast<const Word *>(p));
+      // the lane's last rows of the chunk (fewer than a full group), together
+      Word v[U - 1];
 #pragma unroll
-        for (int q = 0; q < N; ++q)
-          a[q] = op(a[q], ACC(v[q]));
-        p += step;
+      for (int u = 0; u < U - 1; ++u)
+        if (r + down * u < rEnd)
+          v[u] = __builtin_nontemporal_load(reinterpret_cast<const Word *>(p + u * step));
+#pragma unroll
+      for (int q = 0; q < N; ++q) {
+        ACC s[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          s[u] = u < U - 1 && r + down * u < rEnd ? ACC(v[u < U - 1 ? u : 0][q]) : init;
+        a[q] = op(a[q], foldInPairs<U>(s, op));
       }
     }
 #pragma unroll
     for (int q = 0; q < N; ++q)
-      meet[wave][lane * N + q] = a[q];
+      meet[threadIdx.x * N + q] = a[q];
     __syncthreads();
-    for (int c = threadIdx.x; c < NMK_WAVE * N; c += 256) {
-      const int64_t kc = int64_t(blockIdx.x) * NMK_WAVE * N + c;
-      if (kc < nKeep)
-        out[int64_t(blockIdx.y) * nKeep + kc] =
-            op(op(meet[0][c], meet[1][c]), op(meet[2][c], meet[3][c]));
+    for (int half = down / 2; half > 0; half /= 2) {
+      if (int(threadIdx.x >> shift) < half) {
+#pragma unroll
+        for (int q = 0; q < N; ++q)
+          meet[threadIdx.x * N + q] = op(meet[threadIdx.x * N + q],
+                                         meet[(threadIdx.x + (half << shift)) * N + q]);
+      }
+      __syncthreads();
     }
+    const bool direct = gridDim.y == 1;
+    for (int c = threadIdx.x; c < across * N; c += 256) {
+      const int64_t kc = strip0 + c;
+      if (kc < nKeep) {
+        // (a word read further left holds column kc that much later)
+        const int64_t word = kc - c % N;
+        const ACC s = meet[word + N <= nKeep ? c : int(c + (word + N - nKeep))];
+        if (direct)
+          out[kc] = s;
+        else
+          publish(partial + int64_t(blockIdx.y) * nKeep + kc, s);
+      }
+    }
+    if (direct)
+      return;
+    awaitStores();
+    __syncthreads();
+    if (threadIdx.x == 0)
+      isLast = drawLastTicket(stripTicket(tickets, blockIdx.x), gridDim.y) ? 1u : 0u;
+    __syncthreads();
+    if (!isLast)
+      return;
+    // One lane a column while there are lanes enough, several otherwise (of a
+    // strip of at most 128 columns): lane d folds chunks d, d + lanes, ...
+    const int columns = across * N < 256 ? across * N : 256;
+    const int lanes = 256 / columns;
+    for (int c0 = 0; c0 < across * N; c0 += columns) {
+      const int c = c0 + threadIdx.x % columns, d = threadIdx.x / columns;
+      const int64_t kc = strip0 + c;
+      ACC s = init;
+      if (kc < nKeep) {
+        constexpr int F = 16;
+        const ACC *p = partial + kc;
+        const int64_t nChunks = gridDim.y;
+        for (int64_t ch = d; ch < nChunks; ch += F * lanes) {
+          ACC v[F];
+#pragma unroll
+          for (int u = 0; u < F; ++u)
+            v[u] = ch + u * lanes < nChunks ? collect(p + (ch + u * lanes) * nKeep) : init;
+          s = op(s, foldInPairs<F>(v, op));
+        }
+      }
+      __syncthreads(); // (the partial results in meet have been read)
+      meet[threadIdx.x] = s;
+      __syncthreads();
+      if (d == 0 && kc < nKeep) {
+        for (int e = 1; e < lanes; ++e)
+          s = op(s, meet[e * columns + c - c0]);
+        out[kc] = s;
+      }
+    }
+    if (threadIdx.x == 0)
+      publish(stripTicket(tickets, blockIdx.x), 0u);
     return;
   }
   const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -581,9 +674,10 @@ reduceChunks(const IN *__restrict__ x, ACC *__restrict__ out, int64_t n,
   NMK_KERNEL(256)                                                              \
   nmk_reducecols_##OPNAME##_##TNAME(const IN *x, ACC *out, int64_t nRed,       \
                                     int64_t nKeep, int64_t ld,                 \
-                                    int64_t rowsPerChunk, int32_t vec) {       \
-    reduceColumns<IN, ACC>(x, out, nRed, nKeep, ld, rowsPerChunk, vec,         \
-                           ACC(INIT), OP());                                   \
+                                    int64_t rowsPerChunk, int32_t words,       \
+                                    ACC *partial, uint32_t *tickets) {         \
+    reduceColumns<IN, ACC>(x, out, nRed, nKeep, ld, rowsPerChunk, words,       \
+                           partial, tickets, ACC(INIT), OP());                 \
   }                                                                            \
   NMK_KERNEL(256)                                                              \
   nmk_reducechunks_##OPNAME##_##TNAME(const IN *x, ACC *out, int64_t n,        \

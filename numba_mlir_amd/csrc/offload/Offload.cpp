@@ -865,15 +865,24 @@ NMHIP_EXPORT void nmhipReduce(void *ctx, int op, int dtype, const void *x,
     // lanes along the kept index, row chunks over grid.y, partial results
     // folded by the same kernel.
     if (sk == 1 && nKeep > 1 && nRed >= 64 && sr >= nKeep) {
-      // a 128-bit word of adjacent kept indices a lane where every row of
-      // the matrix begins and ends on one
-      const int vec = (aligned16(x) && sr % word == 0 && nKeep % word == 0) ? 1 : 0;
-      const int64_t strips = ceilDiv(nKeep, vec ? 64 * word : 256);
-      // (few long blocks stream best on words -- 256 blocks: 79 us for
-      // [16384, 8192] float32, 2048 blocks: 92 us -- many short ones on
-      // single elements)
-      int64_t chunks =
-          ceilDiv(tuning().colsBlocks ? tuning().colsBlocks : vec ? 256 : 2048, strips);
+      // a 128-bit word of adjacent kept indices a lane (at any element: the
+      // kernel needs no alignment), as many lanes along a row as it has words
+      int across = 0; // log2
+      while (across < 6 && (int64_t(word) << across) < nKeep)
+        ++across;
+      int64_t strips = ceilDiv(nKeep, int64_t(word) << across);
+      const bool words = nKeep >= word && strips <= int64_t(kMaxTickets);
+      if (!words)
+        strips = ceilDiv(nKeep, 256);
+      // (three blocks a CU stream best, measured in us at 256 / 384 / 768 /
+      // 1024 blocks: [5003, 3001] float64 41 / 35 / 34 / 36, [16384, 8192]
+      // float32 96 / 96 / 94 / 118; few strips leave the last blocks many
+      // chunks to fold: [16384, 16] float32 18.9 / 20.7 / 22.4 / 22.5)
+      const int64_t most = tuning().colsBlocks ? tuning().colsBlocks
+                           : !words            ? 2048
+                           : strips < 8        ? 256
+                                               : 768;
+      int64_t chunks = words ? most / strips : ceilDiv(most, strips);
       if (chunks > nRed / 32)
         chunks = nRed / 32;
       if (chunks < 1)
@@ -882,21 +891,18 @@ NMHIP_EXPORT void nmhipReduce(void *ctx, int op, int dtype, const void *x,
         chunks = 65535;
       const int64_t rowsPerChunk = ceilDiv(nRed, chunks);
       chunks = ceilDiv(nRed, rowsPerChunk);
-      if (chunks == 1) {
-        c->launch("nmk_reducecols_" + opAndType, size_t(strips), 1, 1, 256, 1, 1,
-                  {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(nRed), Arg::I64(nKeep),
-                   Arg::I64(sr), Arg::I64(nRed), Arg::I32(vec)});
-      } else {
-        void *partial = c->scratchFor(size_t(chunks) * size_t(nKeep) * accSize);
-        c->launch("nmk_reducecols_" + opAndType, size_t(strips), size_t(chunks), 1,
-                  256, 1, 1,
-                  {Arg::Ptr(x), Arg::Ptr(partial), Arg::I64(nRed), Arg::I64(nKeep),
-                   Arg::I64(sr), Arg::I64(rowsPerChunk), Arg::I32(vec)});
-        c->launch("nmk_reducecols_" + opAndAcc, size_t(ceilDiv(nKeep, 256)), 1, 1, 256, 1,
-                  1,
-                  {Arg::Ptr(partial), Arg::Ptr(out), Arg::I64(chunks),
-                   Arg::I64(nKeep), Arg::I64(nKeep), Arg::I64(chunks), Arg::I32(0)});
-      }
+      const Arg shape = Arg::I32(words ? across + 1 : 0);
+      void *partial =
+          chunks > 1 ? c->scratchFor(size_t(chunks) * size_t(nKeep) * accSize) : nullptr;
+      c->launch("nmk_reducecols_" + opAndType, size_t(strips), size_t(chunks), 1, 256, 1, 1,
+                {Arg::Ptr(x), Arg::Ptr(words || !partial ? out : partial), Arg::I64(nRed),
+                 Arg::I64(nKeep), Arg::I64(sr), Arg::I64(rowsPerChunk), shape,
+                 Arg::Ptr(partial), Arg::Ptr(c->tickets)});
+      if (partial && !words)
+        c->launch("nmk_reducecols_" + opAndAcc, size_t(ceilDiv(nKeep, 256)), 1, 1, 256, 1, 1,
+                  {Arg::Ptr(partial), Arg::Ptr(out), Arg::I64(chunks), Arg::I64(nKeep),
+                   Arg::I64(nKeep), Arg::I64(chunks), Arg::I32(0), Arg::Ptr(nullptr),
+                   Arg::Ptr(nullptr)});
       return;
     }
     // A long contiguous run reduced to one value: a wave per chunk, then the
