@@ -110,6 +110,14 @@ template <> struct Mfma<double> {
 // lies outside it (words are whole: the host checks that the extents along
 // the contiguous dimension are multiples of the word) is read from the
 // operand's first word instead and replaced by zeros.
+//
+// Of an operand contiguous in k, LDS holds element x of row k at
+// x ^ 8 * (k / 2 % 4): 64 lanes write it to eight rows two apart and eight x
+// each, which fall on the same sixteen banks where the rows are laid out
+// straight and on all of them like this; the two rows a half wave reads are
+// moved alike.  (Straight rows: LDS conflicts in 19 % of the cycles, 4096^3
+// 65.3 TFLOP/s with A contiguous in k, 60.6 with both; now 71.4 and 71.0.  An
+// operand contiguous in x is written in whole rows and stays straight.)
 template <int X, bool K_CONTIG, bool GUARD> struct SlabFetch {
   typedef double T;
   typedef Mfma<T> M;
@@ -119,7 +127,7 @@ template <int X, bool K_CONTIG, bool GUARD> struct SlabFetch {
   static constexpr int X_STEP = 256 * M::VEC / BK; // K_CONTIG: x rows per pass
   static constexpr int K_ROWS = 256 * M::VEC / X;     // else: k rows per pass
   static constexpr int WRITES = K_CONTIG ? NV * M::VEC : NV; // LDS instructions
-  int x, k;
+  int x, k, place; // place: the first word's position in its LDS row
   const T *base;
   int64_t ld;
   Vec reg[NV];
@@ -141,7 +149,28 @@ template <int X, bool K_CONTIG, bool GUARD> struct SlabFetch {
       x = (tid % (X / M::VEC)) * M::VEC;
       base = p + int64_t(k) * ld + origin + x;
     }
+    static_assert(!K_CONTIG || X_STEP % 32 == 0, "the words of a thread are moved alike");
+    place = K_CONTIG ? x ^ (8 * (k / 2 % 4)) : x;
     xLeft = extent - origin - x;
+  }
+  // The slab from k0 on, of which `left` of K are left: what lies beyond
+  // counts as zero (the words need not be whole).
+  __device__ __forceinline__ void fetchTail(int k0, int left) {
+    if (left >= BK) {
+      fetch(k0);
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const T *src = K_CONTIG ? base + int64_t(X_STEP * i) * ld + k0
+                              : base + int64_t(k0 + K_ROWS * i) * ld;
+#pragma unroll
+      for (int q = 0; q < M::VEC; ++q) {
+        reg[i][q] = T(0);
+        if (K_CONTIG ? k + q < left : k + K_ROWS * i < left)
+          reg[i][q] = src[q];
+      }
+    }
   }
   __device__ __forceinline__ void fetch(int k0) {
 #pragma unroll
@@ -156,7 +185,9 @@ template <int X, bool K_CONTIG, bool GUARD> struct SlabFetch {
         for (int q = 0; q < M::VEC; ++q)
           reg[i][q] = inside ? v[q] : T(0);
       } else {
-        reg[i] = *reinterpret_cast<const Vec *>(src);
+        // (a tile moved left by an odd number of columns begins inside a word)
+        typedef T Anywhere __attribute__((ext_vector_type(M::VEC), aligned(sizeof(T))));
+        reg[i] = *reinterpret_cast<const Anywhere *>(src);
       }
     }
   }
@@ -168,9 +199,9 @@ template <int X, bool K_CONTIG, bool GUARD> struct SlabFetch {
       if (K_CONTIG) {
 #pragma unroll
         for (int q = 0; q < M::VEC; ++q)
-          lds[k + q][x + X_STEP * i] = reg[i][q];
+          lds[k + q][place + X_STEP * i] = reg[i][q];
       } else {
-        *reinterpret_cast<Vec *>(&lds[k + K_ROWS * i][x]) = reg[i];
+        *reinterpret_cast<Vec *>(&lds[k + K_ROWS * i][place]) = reg[i];
       }
     }
   }
@@ -219,7 +250,10 @@ __host__ __device__ inline int64_t evenSharesStart(int64_t g, int64_t units,
 
 // GUARD: 0 whole tiles; 1 loads and stores guarded (operands and C of any
 // extent); 2 stores alone guarded (operands padded with zeros to whole tiles
-// and slabs, C of any extent).
+// and slabs, C of any extent); 3 M >= BM, N >= BN and otherwise of any extent:
+// the last tiles of a row or column lie further left or up, inside the
+// operands, and store what the tiles before them do not, so that no load but
+// those of the last slab of a K that is not whole slabs is guarded.
 template <int TM, int TN, bool A_KC, bool B_NC, int GUARD>
 __global__ __launch_bounds__(256, 2) void
 dgemm_mfma(const double *__restrict__ A, const double *__restrict__ B, double *__restrict__ C,
@@ -277,8 +311,11 @@ dgemm_mfma(const double *__restrict__ A, const double *__restrict__ B, double *_
 
   SlabFetch<BM, A_KC, GUARD == 1> fa;
   SlabFetch<BN, !B_NC, GUARD == 1> fb;
-  fa.init(A, lda, bm, tid, M, K);
-  fb.init(B, ldb, bn, tid, N, K);
+  // (GUARD 3: how far the tile was moved)
+  const int rowSkip = GUARD == 3 && bm > M - BM ? bm - (M - BM) : 0;
+  const int colSkip = GUARD == 3 && bn > N - BN ? bn - (N - BN) : 0;
+  fa.init(A, lda, bm - rowSkip, tid, M, K);
+  fb.init(B, ldb, bn - colSkip, tid, N, K);
 
   typename MF::Acc acc[TM][TN];
 #pragma unroll
@@ -291,17 +328,27 @@ dgemm_mfma(const double *__restrict__ A, const double *__restrict__ B, double *_
 
   // Operand fragments of one step, double-buffered in registers.
   T a[2][TM], b[2][TN];
+  // (rows kk .. kk + 3 as SlabFetch lays them out)
+  const int moved = xLane ^ (8 * (kLane / 2));
   auto fragments = [&](int stage, int slot, int kk) {
+    const int other = TILE * (kk / MF::KSTEP % 2);
 #pragma unroll
     for (int i = 0; i < TM; ++i)
-      a[slot][i] = As[stage][kk + kLane][wm * (TM * TILE) + i * TILE + xLane];
+      a[slot][i] = As[stage][kk + kLane][wm * (TM * TILE) + ((i * TILE) ^ (A_KC ? other : 0)) +
+                                         (A_KC ? moved : xLane)];
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-      b[slot][j] = Bs[stage][kk + kLane][wn * (TN * TILE) + j * TILE + xLane];
+      b[slot][j] = Bs[stage][kk + kLane][wn * (TN * TILE) + ((j * TILE) ^ (B_NC ? 0 : other)) +
+                                         (B_NC ? xLane : moved)];
   };
 
-  fa.fetch(slab0 * BK);
-  fb.fetch(slab0 * BK);
+  if (GUARD == 3) {
+    fa.fetchTail(slab0 * BK, K - slab0 * BK);
+    fb.fetchTail(slab0 * BK, K - slab0 * BK);
+  } else {
+    fa.fetch(slab0 * BK);
+    fb.fetch(slab0 * BK);
+  }
   fa.stash(As[0]);
   fb.stash(Bs[0]);
   __syncthreads();
@@ -323,13 +370,18 @@ dgemm_mfma(const double *__restrict__ A, const double *__restrict__ B, double *_
   //                   loads have had a third of a slab or more to arrive).
   // The compiler cannot tell the two LDS stages apart, so LDS reads and
   // writes keep their program order: each sits in the step it is issued in.
+  // MORE: 0 the last slab, 1 one before it, 2 the next one may be cut short.
   auto slab = [&](int s, auto more) {
-    constexpr bool MORE = decltype(more)::value;
+    constexpr int NEXT = decltype(more)::value;
+    constexpr bool MORE = NEXT != 0;
     constexpr int STEPS = BK / MF::KSTEP, NMFMA = TM * TN;
     static_assert(STEPS >= 4 && STEPS % 2 == 0, "fragment slots alternate over a slab");
     constexpr int WRITE_STEPS = STEPS / 2 - 1, WRITE_FROM = STEPS - 1 - WRITE_STEPS;
     const int cur = (s - slab0) & 1;
-    if (MORE) {
+    if (NEXT == 2) {
+      fa.fetchTail((s + 1) * BK, K - (s + 1) * BK);
+      fb.fetchTail((s + 1) * BK, K - (s + 1) * BK);
+    } else if (MORE) {
       fa.fetch((s + 1) * BK);
       fb.fetch((s + 1) * BK);
     }
@@ -384,9 +436,12 @@ dgemm_mfma(const double *__restrict__ A, const double *__restrict__ B, double *_
       }
     }
   };
-  for (int s = slab0; s + 1 < slab1; ++s)
-    slab(s, std::true_type());
-  slab(slab1 - 1, std::false_type());
+  int s = slab0;
+  for (; s + (GUARD == 3 ? 2 : 1) < slab1; ++s)
+    slab(s, std::integral_constant<int, 1>());
+  if (GUARD == 3 && s + 1 < slab1)
+    slab(s, std::integral_constant<int, 2>());
+  slab(slab1 - 1, std::integral_constant<int, 0>());
 
   // A whole tile goes to C, scaled; a piece of one goes to its workspace
   // slot as a dense BM x BN block, unscaled.
@@ -406,11 +461,12 @@ dgemm_mfma(const double *__restrict__ A, const double *__restrict__ B, double *_
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const int col = wn * (TN * TILE) + j * TILE + xLane;
+      const int col = wn * (TN * TILE) + j * TILE + xLane - colSkip;
 #pragma unroll
       for (int r = 0; r < MF::NACC; ++r) {
-        const int row = wm * (TM * TILE) + i * TILE + MF::accRow(r, lane);
-        if (GUARD != 0 && !(row < rowsLeft && col < colsLeft))
+        const int row = wm * (TM * TILE) + i * TILE + MF::accRow(r, lane) - rowSkip;
+        if (GUARD == 3 ? row < 0 || col < 0
+                       : GUARD != 0 && !(row < rowsLeft && col < colsLeft))
           continue;
         T *dst = out + int64_t(row) * ldo + col;
         T v = scale * acc[i][j][r];
@@ -1888,6 +1944,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       const bool packX = canPack && offWords(X, ldx, xC);
       const bool packY = canPack && offWords(Y, ldy, yC);
       const bool wordsOk = (packX || !offWords(X, ldx, xC)) && (packY || !offWords(Y, ldy, yC));
+      const bool wordsAligned = !offWords(X, ldx, xC) && !offWords(Y, ldy, yC);
       (void)wordsWhole;
       // Large shapes that are not whole tiles of whole words (256 x 256 for
       // float32, 128 x 128 for float64), where padding them to such tiles
@@ -1899,7 +1956,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       // guarded 128 x 128 tiles in even shares are as fast or faster, 3000^3:
       // 107 against 104), from 256 in float64 (the same tile either way: the
       // copies have to be won back from the guards on the loads alone).
-      bool paddedBig = false;
+      bool paddedBig = false, tilesInside = false;
       {
         constexpr int PT = sizeof(T) == 4 ? 256 : 128;
         const int64_t padSlots = sizeof(T) == 4 ? cus : slots;
@@ -1909,10 +1966,18 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
         const bool fitsAsIs = Mz == Mp && Nz == Np && K % BK == 0 && !offWords(X, ldx, xC) &&
                               !offWords(Y, ldy, yC);
         const int64_t padTiles = (Mp / PT) * (Np / PT);
+        // Operands on the word grid need no copies in float64 where tiles
+        // can be moved inside them (GUARD 3), us with copies / without:
+        // 2000^3 305 / 278, 2400 x 2300 x 1000 235 / 224, 2500 x 2750 x 3000
+        // 722 / 683, 5000 x 5010 x 1000 889 / 867, 7000 x 7500 x 8000 12284 /
+        // 12087.  (From 1.5 to 4 tiles a CU the copies stay: the "+packed" of
+        // nmhipMathLastKernel is relied upon there.)
+        tilesInside = sizeof(T) == 8 && wordsAligned && padTiles >= minTiles && Mz >= 128 &&
+                      Nz >= 128 && (padTiles * 2 < 3 * cus || padTiles > 4 * cus);
         const int slabs = int(Kp / BK);
         int evenBlocks = planEvenShares(padTiles, slabs, padSlots);
-        if (!launched && canPack && !fitsAsIs && (!whole || packX || packY) && K >= 256 &&
-            padTiles >= minTiles &&
+        if (!launched && canPack && !fitsAsIs && !tilesInside && (!whole || packX || packY) &&
+            K >= 256 && padTiles >= minTiles &&
             Mp / PT <= 65535 && Mz <= 0x7fffffff - 256 &&
             Nz <= 0x7fffffff - 256 && K <= 0x7fffffff - 64 &&
             double(Mp) * double(Np) * double(Kp) <= 1.10 * double(Mz) * double(Nz) * double(K)) {
@@ -1985,7 +2050,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       // the GPU then -- 300 x 65536 x 300 float32 15 -> 60 TFLOP/s)
       if (paddedBig || launched) {
         // (done)
-      } else if (((!whole && !onlyK) || packX || packY) && copiesFit && unitOk && wordsOk && K > 0 &&
+      } else if (((!whole && (!onlyK || tilesInside)) || packX || packY) && copiesFit && unitOk && wordsOk && K > 0 &&
           ldx > 0 && ldy > 0 && M <= 0x7fffffff &&
           N <= 0x7fffffff && K <= 0x7fffffff - 64 && tilesM <= 65535 &&
           (tilesM * tilesN >= 16 || (K >= 2048 && Mz * Nz >= 4096))) {
@@ -2035,11 +2100,21 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
         dim3 grid(unsigned(tilesN), unsigned(tilesM), unsigned(plan.slices));
         if (evenBlocks)
           grid = dim3(unsigned(evenBlocks), 1, 1);
+        // (float64: a tile lies inside C, and needs no guards, or C is narrower
+        // than a tile; float32 has one kernel for both)
+        const bool inside = Mz >= 128 && Nz >= 128;
+#define NMHIP_GEMM_RAGGED_(XKC, YNC, GUARD)                                    \
+  hipLaunchKernelGGL((TileKernel<T, 128, XKC, YNC, GUARD>::kernel), grid,      \
+                     dim3(TileKernel<T, 128, XKC, YNC, GUARD>::THREADS), 0,    \
+                     stream, X, Y, cData, int(Mz), int(Nz), int(K), ldxk,      \
+                     ldyk, ldz, alpha, beta, plan.sliceK, W, ldw, even)
 #define NMHIP_GEMM_RAGGED(XKC, YNC)                                            \
-  hipLaunchKernelGGL((TileKernel<T, 128, XKC, YNC, 1>::kernel), grid,          \
-                     dim3(TileKernel<T, 128, XKC, YNC, 1>::THREADS), 0, stream,\
-                     X, Y, cData, int(Mz), int(Nz), int(K), ldxk, ldyk, ldz,   \
-                     alpha, beta, plan.sliceK, W, ldw, even)
+  do {                                                                         \
+    if (inside)                                                                \
+      NMHIP_GEMM_RAGGED_(XKC, YNC, 3);                                         \
+    else                                                                       \
+      NMHIP_GEMM_RAGGED_(XKC, YNC, 1);                                         \
+  } while (0)
         if (xKc && yNc)
           NMHIP_GEMM_RAGGED(true, true);
         else if (xKc)
@@ -2063,6 +2138,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
         else if (plan.slices > 1)
           fold(plan, W, Mz, Nz, ldw, ldz, cData);
 #undef NMHIP_GEMM_RAGGED
+#undef NMHIP_GEMM_RAGGED_
         launched = true;
       } else if (unitOk && mostly && Mt > 0 && Nt > 0 && Kt > 0 &&
           ldx % VEC == 0 && ldy % VEC == 0 && ldx > 0 && ldy > 0 &&

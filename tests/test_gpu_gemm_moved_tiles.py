@@ -1,0 +1,33 @@
+"""GPU parity of float64 products whose last tiles are moved inside the
+operands: extents just above a tile, odd ones, a K that ends inside a slab,
+slices and shares of K, every layout.  Whole numbers: every sum is exact."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ta,tb,tc", [(False, False, False), (True, False, False),
+                                      (False, True, False), (True, True, False),
+                                      (False, False, True), (True, True, True)])
+@pytest.mark.parametrize("m,n,k", [
+    (128, 2050, 18), (2049, 128, 34), (130, 132, 2050),     # one tile across, slices of K
+    (514, 516, 15), (515, 1031, 17), (640, 513, 33),        # odd extents go through copies
+    (1028, 1030, 1026), (1500, 1502, 606),                  # slices, shares
+    (2050, 2052, 270), (2048, 2048, 270),                   # 289 tiles; only K is cut short
+])
+def test_products_of_whole_numbers(hip, m, n, k, ta, tb, tc):
+    from numba_mlir_amd.mlir import math_runtime, ops
+    rng = np.random.default_rng(m + n + k)
+    lay = lambda x, t: hip.asarray(np.ascontiguousarray(x.T)).T if t else hip.asarray(x)
+    a = rng.integers(-99, 99, (m, k), endpoint=True).astype(np.float64)
+    b = rng.integers(-99, 99, (k, n), endpoint=True).astype(np.float64)
+    c0 = rng.integers(-99, 99, (m, n), endpoint=True).astype(np.float64)
+    c = lay(c0.copy(), tc)
+    ops.gemm(lay(a, ta), lay(b, tb), c, 3.0, -2.0)
+    assert "dgemm_mfma_128x128_ragged" in math_runtime.last_kernel()
+    assert np.array_equal(c.asnumpy(), 3.0 * (a @ b) - 2.0 * c0)
+    c = lay(np.full((m, n), np.nan), tc)
+    ops.gemm(lay(a, ta), lay(b, tb), c, 1.0, 0.0)
+    assert np.array_equal(c.asnumpy(), a @ b)
