@@ -234,9 +234,17 @@ template <int MASK> __device__ __forceinline__ void sched_groups(int n) {
 // gemm_even_fold adds a tile's pieces in K order.  Used when whole tiles
 // would leave the last round of blocks mostly empty (576 tiles on 256 CUs:
 // 2.25 rounds) or would not fill the first.
+//
+// Of many rounds, all but the last whole one and the rest behind it run as
+// whole tiles, block g taking tiles g, g + G, ... below `whole`: the blocks
+// then work side by side on neighbouring tiles, which share their operands in
+// the caches, and only one to two rounds of tiles are dealt out in shares
+// (us with every tile dealt out / with this: float64 6000 x 6002 x 302 473 /
+// 434, 6000 x 5800 x 3000 3246 / 3081, float32 6144 x 6144 x 256 197 / 181).
 struct EvenShares {
-  int slabs;  // K slabs a tile (0: not in use)
-  int tilesN; // block tiles along N
+  int slabs;   // K slabs a tile (0: not in use)
+  int tilesN;  // block tiles along N
+  int64_t whole; // tiles that come before the shares, a block each
 };
 __host__ __device__ inline int64_t evenSharesStart(int64_t g, int64_t units,
                                                    int64_t blocks) {
@@ -284,30 +292,40 @@ dgemm_mfma(const double *__restrict__ A, const double *__restrict__ B, double *_
 
   // This block's units (one segment, the whole of K of one tile, without
   // even shares).
-  int64_t unit = 0, unitEnd = 0;
+  int64_t unit = 0, unitEnd = 0, wholeTile = blockIdx.x;
   const int slabsPerTile = even.slabs > 0 ? even.slabs : (K + BK - 1) / BK;
   if (even.slabs > 0) {
-    const int64_t units = int64_t((M + BM - 1) / BM) * even.tilesN * even.slabs;
+    const int64_t units =
+        (int64_t((M + BM - 1) / BM) * even.tilesN - even.whole) * even.slabs;
     unit = evenSharesStart(blockIdx.x, units, gridDim.x);
     unitEnd = evenSharesStart(int64_t(blockIdx.x) + 1, units, gridDim.x);
   } else {
     unitEnd = slabsPerTile;
   }
 #pragma nounroll
-  for (int segment = 0; unit < unitEnd; ++segment) {
+  for (int segment = 0; unit < unitEnd; ) {
   int bm = blockIdx.y * BM, bn = blockIdx.x * BN;
   int slab0 = 0, slab1 = slabsPerTile; // the K slabs of this segment
+  const bool shared = wholeTile >= even.whole; // (else a tile before the shares)
   if (even.slabs > 0) {
-    const int64_t tile = unit / even.slabs;
-    slab0 = int(unit - tile * even.slabs);
-    slab1 = unitEnd - unit < even.slabs - slab0 ? slab0 + int(unitEnd - unit) : even.slabs;
+    int64_t tile = wholeTile;
+    if (shared) {
+      tile = unit / even.slabs;
+      slab0 = int(unit - tile * even.slabs);
+      slab1 = unitEnd - unit < even.slabs - slab0 ? slab0 + int(unitEnd - unit) : even.slabs;
+      tile += even.whole;
+    }
     bm = int(tile / even.tilesN) * BM;
     bn = int(tile % even.tilesN) * BN;
-    if (segment > 0)
-      __syncthreads(); // every wave is done with the last segment's LDS slabs
+    __syncthreads(); // every wave is done with the last segment's LDS slabs
   }
-  unit += slab1 - slab0;
   const bool piece = even.slabs > 0 && !(slab0 == 0 && slab1 == even.slabs);
+  const int slot = segment > 0 ? 1 : 0;
+  if (shared) {
+    unit += slab1 - slab0;
+    ++segment;
+  }
+  wholeTile += gridDim.x;
 
   SlabFetch<BM, A_KC, GUARD == 1> fa;
   SlabFetch<BN, !B_NC, GUARD == 1> fb;
@@ -450,7 +468,7 @@ dgemm_mfma(const double *__restrict__ A, const double *__restrict__ B, double *_
   T scale = alpha, keep = beta;
   int rowsLeft = GUARD != 0 ? M - bm : BM, colsLeft = GUARD != 0 ? N - bn : BN;
   if (piece) {
-    out = W + (int64_t(blockIdx.x) * 2 + (segment > 0 ? 1 : 0)) * (BM * BN);
+    out = W + (int64_t(blockIdx.x) * 2 + slot) * (BM * BN);
     ldo = BN;
     scale = T(1);
     keep = T(0);
@@ -511,7 +529,7 @@ template <bool A_KC, bool B_NC, int GUARD> struct TileKernel<double, 128, A_KC, 
 template <typename T, int BM, int BN>
 __global__ __launch_bounds__(256) void
 gemm_even_fold(const T *__restrict__ W, int64_t blocks, int slabs, int tilesN,
-               int64_t units, T *__restrict__ C, int M, int N, int64_t ldc,
+               int64_t whole, int64_t units, T *__restrict__ C, int M, int N, int64_t ldc,
                T alpha, T beta) {
   typedef typename Mfma<T>::Vec Vec;
   constexpr int VEC = Mfma<T>::VEC;
@@ -542,7 +560,8 @@ gemm_even_fold(const T *__restrict__ W, int64_t blocks, int slabs, int tilesN,
     const T *slot = W + (g * 2 + (b >= u0 ? 0 : 1)) * int64_t(BM * BN);
     sum += *reinterpret_cast<const Vec *>(slot + row * BN + col);
   }
-  const int gr = int(tile / tilesN) * BM + row, gc = int(tile % tilesN) * BN + col;
+  const int gr = int((whole + tile) / tilesN) * BM + row;
+  const int gc = int((whole + tile) % tilesN) * BN + col;
   if (gr >= M)
     return;
   T *dst = C + int64_t(gr) * ldc + gc;
@@ -1396,19 +1415,35 @@ SplitPlan planSplit(int64_t tiles, int64_t K, int BK, int64_t slots /* resident 
 }
 
 // Blocks of an even-shares launch over `tiles` block tiles of `slabs` K slabs
-// each on `slots` resident blocks, or 0 when whole tiles do as well: they
-// fill their rounds to nine tenths or more, or a block's share would be under
-// eight slabs (the pieces' trip through the workspace would cost more than
-// the idle CUs).
-int planEvenShares(int64_t tiles, int64_t slabs, int64_t slots) {
+// each on `slots` resident blocks, perCu of them a CU, or 0 when whole tiles do
+// as well: they fill their rounds to nine tenths or more, or a block's share
+// would be under eight slabs (the pieces' trip through the workspace would
+// cost more than the idle CUs).  Where two blocks share a CU, one that is
+// left alone there in the last round runs nearly twice as fast: whole tiles
+// in shares / as they are, us: 7000 x 7500 x 8000 float64, rounds filled to
+// 0.905, 12150 / 12061.  One block a CU gains up to a fill of 0.95 (8000 x
+// 7500 x 7000 float32, 0.94: 3972 / 4080; measured to four rounds).
+int planEvenShares(int64_t tiles, int64_t slabs, int64_t slots, int perCu) {
   if (tiles <= 0 || slabs <= 0)
     return 0;
   const int64_t rounds = (tiles + slots - 1) / slots;
-  if (tiles * 10 >= rounds * slots * 9)
+  const int64_t enough = perCu == 1 && rounds <= 4 ? 95 : 90;
+  if (tiles * 100 >= rounds * slots * enough)
     return 0;
   if (tiles * slabs < 8 * slots)
     return 0;
   return int(slots);
+}
+
+// Tiles of an even-shares launch of `blocks` blocks that are not dealt out: all
+// whole rounds but the last.
+int64_t wholeBeforeShares(int64_t tiles, int64_t blocks) {
+  return tiles >= 2 * blocks ? (tiles / blocks - 1) * blocks : 0;
+}
+EvenShares sharesOf(int blocks, int slabs, int64_t tiles, int64_t tilesN) {
+  if (blocks <= 0)
+    return EvenShares{0, int(tilesN), 0};
+  return EvenShares{slabs, int(tilesN), wholeBeforeShares(tiles, blocks)};
 }
 
 // Whether cutting K into plan.slices equal slices goes ahead of even shares:
@@ -1602,15 +1637,16 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
 
   auto evenFold = [&](const T *W, int blocks, int slabs, int64_t tilesM, int64_t tilesN,
                       int tile, int64_t m, int64_t n, int64_t ldz, T *Z) {
-    const int64_t units = tilesM * tilesN * slabs;
-    dim3 grid(unsigned(tilesM * tilesN), unsigned(tile * tile / Mfma<T>::VEC / 256));
+    const int64_t whole = wholeBeforeShares(tilesM * tilesN, blocks);
+    const int64_t tiles = tilesM * tilesN - whole, units = tiles * slabs;
+    dim3 grid(unsigned(tiles), unsigned(tile * tile / Mfma<T>::VEC / 256));
     if (tile == 256)
       hipLaunchKernelGGL((gemm_even_fold<T, 256, 256>), grid, dim3(256), 0, stream, W,
-                         int64_t(blocks), slabs, int(tilesN), units, Z, int(m), int(n),
+                         int64_t(blocks), slabs, int(tilesN), whole, units, Z, int(m), int(n),
                          ldz, alpha, beta);
     else
       hipLaunchKernelGGL((gemm_even_fold<T, 128, 128>), grid, dim3(256), 0, stream, W,
-                         int64_t(blocks), slabs, int(tilesN), units, Z, int(m), int(n),
+                         int64_t(blocks), slabs, int(tilesN), whole, units, Z, int(m), int(n),
                          ldz, alpha, beta);
   };
 
@@ -1893,7 +1929,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       const bool bigFits = sizeof(T) == 4 && Mt % 256 == 0 && Nt % 256 == 0;
       const int64_t bigTiles = (Mt / 256) * (Nt / 256);
       const int bigEven = bigFits && workspaceKind == WORKSPACE_HEAP
-                              ? planEvenShares(bigTiles, Kt / BK, cus)
+                              ? planEvenShares(bigTiles, Kt / BK, cus, 1)
                               : 0;
       // (from 64 large tiles on: below, the 128 x 128 tiles in slices or
       // shares are as fast or faster -- 1792^3 120 against 131 us, 1024 x
@@ -1975,7 +2011,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
         tilesInside = sizeof(T) == 8 && wordsAligned && padTiles >= minTiles && Mz >= 128 &&
                       Nz >= 128 && (padTiles * 2 < 3 * cus || padTiles > 4 * cus);
         const int slabs = int(Kp / BK);
-        int evenBlocks = planEvenShares(padTiles, slabs, padSlots);
+        int evenBlocks = planEvenShares(padTiles, slabs, padSlots, int(padSlots / cus));
         if (!launched && canPack && !fitsAsIs && !tilesInside && (!whole || packX || packY) &&
             K >= 256 && padTiles >= minTiles &&
             Mp / PT <= 65535 && Mz <= 0x7fffffff - 256 &&
@@ -2004,7 +2040,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
             T *Xp = reinterpret_cast<T *>(base), *Yp = reinterpret_cast<T *>(base + xBytes);
             pack(X, ldx, xR, xC, xRp, xCp, Xp);
             pack(Y, ldy, yR, yC, yRp, yCp, Yp);
-            const EvenShares even{evenBlocks ? slabs : 0, int(Np / PT)};
+            const EvenShares even = sharesOf(evenBlocks, slabs, padTiles, Np / PT);
             dim3 grid(unsigned(Np / PT), unsigned(Mp / PT), 1);
             if (evenBlocks)
               grid = dim3(unsigned(evenBlocks), 1, 1);
@@ -2062,7 +2098,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
         bool slicesFill = false;
         SplitPlan plan = planSlices(tilesM * tilesN, K, slicesFill);
         int evenBlocks = workspaceKind == WORKSPACE_HEAP && !slicesFill
-                             ? planEvenShares(tilesM * tilesN, slabs, slots)
+                             ? planEvenShares(tilesM * tilesN, slabs, slots, 2)
                              : 0;
         T *W = evenWorkspace(evenBlocks, 128, 128);
         if (evenBlocks)
@@ -2096,7 +2132,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
           }
         }
         const int64_t ldxk = packX ? xCp : ldx, ldyk = packY ? yCp : ldy;
-        const EvenShares even{evenBlocks ? slabs : 0, int(tilesN)};
+        const EvenShares even = sharesOf(evenBlocks, slabs, tilesM * tilesN, tilesN);
         dim3 grid(unsigned(tilesN), unsigned(tilesM), unsigned(plan.slices));
         if (evenBlocks)
           grid = dim3(unsigned(evenBlocks), 1, 1);
@@ -2151,7 +2187,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
           plan = planSlices((Mt / BM) * (Nt / BN), Kt, slicesFill);
         int evenBlocks = big ? bigEven
                          : workspaceKind == WORKSPACE_HEAP && !slicesFill
-                             ? planEvenShares((Mt / BM) * (Nt / BN), slabs, slots)
+                             ? planEvenShares((Mt / BM) * (Nt / BN), slabs, slots, 2)
                              : 0;
         T *W = evenWorkspace(evenBlocks, BM, BN);
         if (evenBlocks)
@@ -2160,7 +2196,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
           W = workspaceFor(plan, Mt, Nt, true);
         if (tooLarge)
           return 1;
-        const EvenShares even{evenBlocks ? slabs : 0, int(Nt / BN)};
+        const EvenShares even = sharesOf(evenBlocks, slabs, (Mt / BM) * (Nt / BN), Nt / BN);
         dim3 grid(unsigned(Nt / BN), unsigned(Mt / BM), unsigned(plan.slices));
         if (evenBlocks)
           grid = dim3(unsigned(evenBlocks), 1, 1);

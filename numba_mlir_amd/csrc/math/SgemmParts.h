@@ -235,30 +235,40 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
   const int aWord = wm * (TM * 32) + lane % 32 + lane / 32 * PartsSlab<BM>::HALF;
   const int bWord = wn * (TN * 32) + lane % 32 + lane / 32 * PartsSlab<BN>::HALF;
 
-  int64_t unit = 0, unitEnd = 0;
+  int64_t unit = 0, unitEnd = 0, wholeTile = blockIdx.x;
   const int slabsPerTile = even.slabs > 0 ? even.slabs : (K + BK - 1) / BK;
   if (even.slabs > 0) {
-    const int64_t units = int64_t((M + BM - 1) / BM) * even.tilesN * even.slabs;
+    const int64_t units =
+        (int64_t((M + BM - 1) / BM) * even.tilesN - even.whole) * even.slabs;
     unit = evenSharesStart(blockIdx.x, units, gridDim.x);
     unitEnd = evenSharesStart(int64_t(blockIdx.x) + 1, units, gridDim.x);
   } else {
     unitEnd = slabsPerTile;
   }
 #pragma nounroll
-  for (int segment = 0; unit < unitEnd; ++segment) {
+  for (int segment = 0; unit < unitEnd; ) {
     int bm = blockIdx.y * BM, bn = blockIdx.x * BN;
     int slab0 = 0, slab1 = slabsPerTile; // the K slabs of this segment
+    const bool shared = wholeTile >= even.whole; // (else a tile before the shares)
     if (even.slabs > 0) {
-      const int64_t tile = unit / even.slabs;
-      slab0 = int(unit - tile * even.slabs);
-      slab1 = unitEnd - unit < even.slabs - slab0 ? slab0 + int(unitEnd - unit) : even.slabs;
+      int64_t tile = wholeTile;
+      if (shared) {
+        tile = unit / even.slabs;
+        slab0 = int(unit - tile * even.slabs);
+        slab1 = unitEnd - unit < even.slabs - slab0 ? slab0 + int(unitEnd - unit) : even.slabs;
+        tile += even.whole;
+      }
       bm = int(tile / even.tilesN) * BM;
       bn = int(tile % even.tilesN) * BN;
-      if (segment > 0)
-        __syncthreads(); // every wave is done with the last segment's LDS slabs
+      __syncthreads(); // every wave is done with the last segment's LDS slabs
     }
-    unit += slab1 - slab0;
     const bool piece = even.slabs > 0 && !(slab0 == 0 && slab1 == even.slabs);
+    const int slot = segment > 0 ? 1 : 0;
+    if (shared) {
+      unit += slab1 - slab0;
+      ++segment;
+    }
+    wholeTile += gridDim.x;
 
     PartsFetch<BM, A_KC, THREADS> fa;
     PartsFetch<BN, !B_NC, THREADS> fb;
@@ -403,7 +413,7 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
     float scale = alpha, keep = beta;
     int rowsLeft = M - bm, colsLeft = N - bn;
     if (piece) {
-      out = W + (int64_t(blockIdx.x) * 2 + (segment > 0 ? 1 : 0)) * (BM * BN);
+      out = W + (int64_t(blockIdx.x) * 2 + slot) * (BM * BN);
       ldo = BN;
       scale = 1.0f;
       keep = 0.0f;
