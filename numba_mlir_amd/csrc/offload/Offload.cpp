@@ -423,6 +423,16 @@ public:
         retireEvent(ev, true);
   }
 
+  // A result of a few bytes that a launch leaves straight in the pinned block:
+  // one launch and one wait, where a copy from device memory is a second of
+  // each (a float32 norm through njit 41 -> 20 us).
+  template <typename Launch> void resultToHost(void *host, size_t bytes, Launch launchInto) {
+    char *stage = stagingHalf(0);
+    launchInto(static_cast<void *>(stage));
+    synchronize(); // (an asynchronous context's launch)
+    std::memcpy(host, stage, bytes);
+  }
+
   void deviceToHost(void *host, const void *dev, size_t bytes) {
     synchronize();
     void *pending[2] = {nullptr, nullptr};
@@ -763,192 +773,231 @@ NMHIP_EXPORT void nmhipBlackScholesF32(void *ctx, const float *price,
   });
 }
 
+namespace {
+
+// The reduction into `out` (device memory, or pinned host memory, which the
+// kernels only store to); the context's mutex is held.
+void reduceInto(Context *c, int op, int dtype, const void *x, int64_t n0, int64_t n1,
+                int64_t s0, int64_t s1, int axis, void *out) {
+  if (n0 < 0 || n1 < 0)
+    fail("nmhipReduce: negative extent");
+  if (axis < -1 || axis > 1)
+    fail("nmhipReduce: axis must be -1, 0 or 1");
+  static const char *const opNames[] = {"sum", "prod", "min", "max"};
+  if (op < 0 || op > NMHIP_MAX)
+    fail("Unsupported reduce op %d", op);
+  const bool rowMajor = s1 == 1 && (n0 <= 1 || s0 >= n1);
+  const bool contiguous = s1 == 1 && (n0 <= 1 || s0 == n1);
+
+  // float32 row sums: a wave per row.
+  if (op == NMHIP_SUM && dtype == NMHIP_F32 && axis == 1 && rowMajor &&
+      n0 > 0 && n1 > 0) {
+    const int vec = (aligned16(x) && s0 % 4 == 0 && n1 % 4 == 0) ? 1 : 0;
+    // a block per row for long rows, a wave per row otherwise
+    const bool wide = n1 >= 4096;
+    c->launchBlocksXY(wide ? wideRowKernel("nmk_sum_axis1", n0, n1, vec != 0)
+                           : std::string("nmk_sum_axis1_f32"),
+                      wide ? n0 : ceilDiv(n0, 4),
+                      {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(n0), Arg::I64(n1),
+                       Arg::I64(s0), Arg::I32(vec)});
+    return;
+  }
+  // int32 column sums into int64: column strips x row chunks, device finish.
+  if (op == NMHIP_SUM && dtype == NMHIP_I32 && axis == 0 && rowMajor &&
+      aligned16(x) && s0 % 4 == 0 && n1 % 4 == 0 && n0 >= 64 && n1 > 0) {
+    const int64_t strips = ceilDiv(n1, 256);
+    int64_t rowsPerBlock = tuning().axis0Rows;
+    if (!rowsPerBlock) {
+      // One block per CU (256) measured fastest: few, long-lived blocks
+      // keep the finish short.  Chunks of whole 64 rows: at [16384, 8192]
+      // they start 64 MiB apart, which measured 2 us faster than chunks of
+      // whole 24-row groups (6 loads x 4 waves) that do not.
+      rowsPerBlock = ceilDiv(n0 * strips, 256);
+      rowsPerBlock = ceilDiv(rowsPerBlock, 64) * 64;
+    }
+    const int64_t chunks = ceilDiv(n0, rowsPerBlock);
+    if (strips <= int64_t(kMaxTickets) && chunks <= 65535) {
+      void *partial = c->scratchFor(size_t(chunks) * size_t(n1) * 8);
+      c->launch("nmk_sum_axis0_i32_i64", size_t(strips), size_t(chunks), 1,
+                256, 1, 1,
+                {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(n0), Arg::I64(n1),
+                 Arg::I64(s0), Arg::I64(rowsPerBlock), Arg::Ptr(partial),
+                 Arg::Ptr(c->tickets)});
+      return;
+    }
+  }
+  // float32 full sum: grid-stride, device finish.
+  if (op == NMHIP_SUM && dtype == NMHIP_F32 && axis == -1 && contiguous &&
+      n0 * n1 >= 4096) {
+    const int64_t n = n0 * n1;
+    int64_t blocks = tuning().reduceBlocks ? tuning().reduceBlocks : kFullSumBlocks;
+    const int64_t need = ceilDiv(n, 256 * 16);
+    if (blocks > need)
+      blocks = need;
+    void *partial = c->scratchFor(size_t(blocks) * 4);
+    c->launch("nmk_sum_all_f32", size_t(blocks), 1, 1, 256, 1, 1,
+              {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(n),
+               Arg::I32(aligned16(x) ? 1 : 0), Arg::Ptr(partial),
+               Arg::Ptr(c->tickets)});
+    return;
+  }
+  // Generic strided fallback: a wave per kept index.
+  int64_t nKeep, nRed, sk, sr;
+  if (axis == 1) {
+    nKeep = n0;
+    nRed = n1;
+    sk = s0;
+    sr = s1;
+  } else if (axis == 0) {
+    nKeep = n1;
+    nRed = n0;
+    sk = s1;
+    sr = s0;
+  } else {
+    if (!contiguous)
+      fail("nmhipReduce: a full reduction needs a C-contiguous array");
+    nKeep = 1;
+    nRed = n0 * n1;
+    sk = 0;
+    sr = 1;
+  }
+  if (nKeep == 0)
+    return;
+  const std::string opAndType = std::string(opNames[op]) + "_" + dtypeName(dtype);
+  // the accumulator type's own kernels fold partial results
+  const bool isInt = dtype == NMHIP_I32 || dtype == NMHIP_I64;
+  const std::string opAndAcc =
+      std::string(opNames[op]) + "_" + (isInt ? "i64" : dtypeName(dtype));
+  const size_t accSize = dtype == NMHIP_F32 ? 4 : 8;
+  // elements of the input in a 128-bit word
+  const int64_t word = (dtype == NMHIP_F32 || dtype == NMHIP_I32) ? 4 : 2;
+  // The kept index has unit stride (column sums of a row-major matrix):
+  // lanes along the kept index, row chunks over grid.y, partial results
+  // folded by the same kernel.
+  if (sk == 1 && nKeep > 1 && nRed >= 64 && sr >= nKeep) {
+    // a 128-bit word of adjacent kept indices a lane (at any element: the
+    // kernel needs no alignment), as many lanes along a row as it has words
+    int across = 0; // log2
+    while (across < 6 && (int64_t(word) << across) < nKeep)
+      ++across;
+    int64_t strips = ceilDiv(nKeep, int64_t(word) << across);
+    const bool words = nKeep >= word && strips <= int64_t(kMaxTickets);
+    if (!words)
+      strips = ceilDiv(nKeep, 256);
+    // (three blocks a CU stream best, measured in us at 256 / 384 / 768 /
+    // 1024 blocks: [5003, 3001] float64 41 / 35 / 34 / 36, [16384, 8192]
+    // float32 96 / 96 / 94 / 118; few strips leave the last blocks many
+    // chunks to fold: [16384, 16] float32 18.9 / 20.7 / 22.4 / 22.5)
+    const int64_t most = tuning().colsBlocks ? tuning().colsBlocks
+                         : !words            ? 2048
+                         : strips < 8        ? 256
+                                             : 768;
+    int64_t chunks = words ? most / strips : ceilDiv(most, strips);
+    if (chunks > nRed / 32)
+      chunks = nRed / 32;
+    if (chunks < 1)
+      chunks = 1;
+    if (chunks > 65535)
+      chunks = 65535;
+    const int64_t rowsPerChunk = ceilDiv(nRed, chunks);
+    chunks = ceilDiv(nRed, rowsPerChunk);
+    const Arg shape = Arg::I32(words ? across + 1 : 0);
+    void *partial =
+        chunks > 1 ? c->scratchFor(size_t(chunks) * size_t(nKeep) * accSize) : nullptr;
+    c->launch("nmk_reducecols_" + opAndType, size_t(strips), size_t(chunks), 1, 256, 1, 1,
+              {Arg::Ptr(x), Arg::Ptr(words || !partial ? out : partial), Arg::I64(nRed),
+               Arg::I64(nKeep), Arg::I64(sr), Arg::I64(rowsPerChunk), shape,
+               Arg::Ptr(partial), Arg::Ptr(c->tickets)});
+    if (partial && !words)
+      c->launch("nmk_reducecols_" + opAndAcc, size_t(ceilDiv(nKeep, 256)), 1, 1, 256, 1, 1,
+                {Arg::Ptr(partial), Arg::Ptr(out), Arg::I64(chunks), Arg::I64(nKeep),
+                 Arg::I64(nKeep), Arg::I64(chunks), Arg::I32(0), Arg::Ptr(nullptr),
+                 Arg::Ptr(nullptr)});
+    return;
+  }
+  // A long contiguous run reduced to one value: a wave per chunk, then the
+  // chunks' results by one wave.
+  if (nKeep == 1 && sr == 1 && nRed >= 65536) {
+    // one block a chunk: as many as stream well at once, 16 KiB or more each
+    int64_t nChunks = ceilDiv(nRed * int64_t(16 / word), 16384);
+    const int64_t most = tuning().reduceBlocks ? tuning().reduceBlocks : 512;
+    if (nChunks > most)
+      nChunks = most;
+    // (chunks of whole 128-bit words, so that every chunk of an aligned
+    // array starts on one)
+    const int64_t chunk = ceilDiv(ceilDiv(nRed, nChunks), word) * word;
+    nChunks = ceilDiv(nRed, chunk);
+    void *partial = c->scratchFor(size_t(nChunks) * accSize);
+    c->launch("nmk_reducechunks_" + opAndType, size_t(nChunks), 1, 1, 256, 1, 1,
+              {Arg::Ptr(x), Arg::Ptr(partial), Arg::I64(nRed), Arg::I64(chunk),
+               Arg::I64(nChunks), Arg::I32(aligned16(x) ? 1 : 0)});
+    c->launch("nmk_reduce_" + opAndAcc, 1, 1, 1, 256, 1, 1,
+              {Arg::Ptr(partial), Arg::Ptr(out), Arg::I64(1), Arg::I64(nChunks),
+               Arg::I64(0), Arg::I64(1), Arg::I64(1), Arg::I32(0)});
+    return;
+  }
+  // Many short runs (the rows of a tall matrix of a few columns): a group
+  // of 1 to 32 lanes a kept index, two elements or so a lane.
+  if (nRed >= 1 && nRed <= 64 && nKeep >= 4096) {
+    int gShift = 0;
+    while (sr == 1 && (int64_t(2) << gShift) < nRed && gShift < 5)
+      ++gShift; // (a lane a kept index where the run is strided: the lanes then
+                // follow the kept index, which has the shorter stride)
+    const int mode = 4 | (gShift << 8);
+    c->launchBlocksXY(std::string("nmk_reduce_") + opNames[op] + "_" + dtypeName(dtype),
+                      ceilDiv(nKeep << gShift, 256),
+                      {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(nKeep), Arg::I64(nRed),
+                       Arg::I64(sk), Arg::I64(sr), Arg::I64(1), Arg::I32(mode)});
+    return;
+  }
+  // (a block per kept index where the reduced run is long, a wave per
+  // kept index otherwise)
+  const bool wide = nRed >= 4096;
+  const int mode = ((sr == 1 && aligned16(x) && (nKeep == 1 || sk % word == 0)) ? 1 : 0) |
+                   (wide ? 2 : 0);
+  c->launchBlocksXY(std::string("nmk_reduce_") + opNames[op] + "_" + dtypeName(dtype),
+                    wide ? nKeep : ceilDiv(nKeep, 4),
+                    {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(nKeep), Arg::I64(nRed),
+                     Arg::I64(sk), Arg::I64(sr), Arg::I64(1), Arg::I32(mode)});
+}
+
+void norm2Into(Context *c, const float *x, int64_t n, float *out) {
+  if (n < 0)
+    fail("nmhipNorm2F32: negative extent");
+  int64_t blocks = tuning().reduceBlocks ? tuning().reduceBlocks : kFullSumBlocks;
+  int64_t need = ceilDiv(n, 256 * 16);
+  if (need < 1)
+    need = 1;
+  if (blocks > need)
+    blocks = need;
+  void *partial = c->scratchFor(size_t(blocks) * 4);
+  c->launch("nmk_norm2_f32", size_t(blocks), 1, 1, 256, 1, 1,
+            {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(n),
+             Arg::I32(aligned16(x) ? 1 : 0), Arg::Ptr(partial),
+             Arg::Ptr(c->tickets)});
+}
+
+} // namespace
+
 NMHIP_EXPORT void nmhipReduce(void *ctx, int op, int dtype, const void *x,
                               int64_t n0, int64_t n1, int64_t s0, int64_t s1,
                               int axis, void *out) {
   guarded([&]() {
     Context *c = toCtx(ctx);
     std::lock_guard<std::mutex> lock(c->mutex);
-    if (n0 < 0 || n1 < 0)
-      fail("nmhipReduce: negative extent");
-    if (axis < -1 || axis > 1)
-      fail("nmhipReduce: axis must be -1, 0 or 1");
-    static const char *const opNames[] = {"sum", "prod", "min", "max"};
-    if (op < 0 || op > NMHIP_MAX)
-      fail("Unsupported reduce op %d", op);
-    const bool rowMajor = s1 == 1 && (n0 <= 1 || s0 >= n1);
-    const bool contiguous = s1 == 1 && (n0 <= 1 || s0 == n1);
+    reduceInto(c, op, dtype, x, n0, n1, s0, s1, axis, out);
+  });
+}
 
-    // float32 row sums: a wave per row.
-    if (op == NMHIP_SUM && dtype == NMHIP_F32 && axis == 1 && rowMajor &&
-        n0 > 0 && n1 > 0) {
-      const int vec = (aligned16(x) && s0 % 4 == 0 && n1 % 4 == 0) ? 1 : 0;
-      // a block per row for long rows, a wave per row otherwise
-      const bool wide = n1 >= 4096;
-      c->launchBlocksXY(wide ? wideRowKernel("nmk_sum_axis1", n0, n1, vec != 0)
-                             : std::string("nmk_sum_axis1_f32"),
-                        wide ? n0 : ceilDiv(n0, 4),
-                        {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(n0), Arg::I64(n1),
-                         Arg::I64(s0), Arg::I32(vec)});
-      return;
-    }
-    // int32 column sums into int64: column strips x row chunks, device finish.
-    if (op == NMHIP_SUM && dtype == NMHIP_I32 && axis == 0 && rowMajor &&
-        aligned16(x) && s0 % 4 == 0 && n1 % 4 == 0 && n0 >= 64 && n1 > 0) {
-      const int64_t strips = ceilDiv(n1, 256);
-      int64_t rowsPerBlock = tuning().axis0Rows;
-      if (!rowsPerBlock) {
-        // One block per CU (256) measured fastest: few, long-lived blocks
-        // keep the finish short.  Chunks of whole 64 rows: at [16384, 8192]
-        // they start 64 MiB apart, which measured 2 us faster than chunks of
-        // whole 24-row groups (6 loads x 4 waves) that do not.
-        rowsPerBlock = ceilDiv(n0 * strips, 256);
-        rowsPerBlock = ceilDiv(rowsPerBlock, 64) * 64;
-      }
-      const int64_t chunks = ceilDiv(n0, rowsPerBlock);
-      if (strips <= int64_t(kMaxTickets) && chunks <= 65535) {
-        void *partial = c->scratchFor(size_t(chunks) * size_t(n1) * 8);
-        c->launch("nmk_sum_axis0_i32_i64", size_t(strips), size_t(chunks), 1,
-                  256, 1, 1,
-                  {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(n0), Arg::I64(n1),
-                   Arg::I64(s0), Arg::I64(rowsPerBlock), Arg::Ptr(partial),
-                   Arg::Ptr(c->tickets)});
-        return;
-      }
-    }
-    // float32 full sum: grid-stride, device finish.
-    if (op == NMHIP_SUM && dtype == NMHIP_F32 && axis == -1 && contiguous &&
-        n0 * n1 >= 4096) {
-      const int64_t n = n0 * n1;
-      int64_t blocks = tuning().reduceBlocks ? tuning().reduceBlocks : kFullSumBlocks;
-      const int64_t need = ceilDiv(n, 256 * 16);
-      if (blocks > need)
-        blocks = need;
-      void *partial = c->scratchFor(size_t(blocks) * 4);
-      c->launch("nmk_sum_all_f32", size_t(blocks), 1, 1, 256, 1, 1,
-                {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(n),
-                 Arg::I32(aligned16(x) ? 1 : 0), Arg::Ptr(partial),
-                 Arg::Ptr(c->tickets)});
-      return;
-    }
-    // Generic strided fallback: a wave per kept index.
-    int64_t nKeep, nRed, sk, sr;
-    if (axis == 1) {
-      nKeep = n0;
-      nRed = n1;
-      sk = s0;
-      sr = s1;
-    } else if (axis == 0) {
-      nKeep = n1;
-      nRed = n0;
-      sk = s1;
-      sr = s0;
-    } else {
-      if (!contiguous)
-        fail("nmhipReduce: a full reduction needs a C-contiguous array");
-      nKeep = 1;
-      nRed = n0 * n1;
-      sk = 0;
-      sr = 1;
-    }
-    if (nKeep == 0)
-      return;
-    const std::string opAndType = std::string(opNames[op]) + "_" + dtypeName(dtype);
-    // the accumulator type's own kernels fold partial results
-    const bool isInt = dtype == NMHIP_I32 || dtype == NMHIP_I64;
-    const std::string opAndAcc =
-        std::string(opNames[op]) + "_" + (isInt ? "i64" : dtypeName(dtype));
-    const size_t accSize = dtype == NMHIP_F32 ? 4 : 8;
-    // elements of the input in a 128-bit word
-    const int64_t word = (dtype == NMHIP_F32 || dtype == NMHIP_I32) ? 4 : 2;
-    // The kept index has unit stride (column sums of a row-major matrix):
-    // lanes along the kept index, row chunks over grid.y, partial results
-    // folded by the same kernel.
-    if (sk == 1 && nKeep > 1 && nRed >= 64 && sr >= nKeep) {
-      // a 128-bit word of adjacent kept indices a lane (at any element: the
-      // kernel needs no alignment), as many lanes along a row as it has words
-      int across = 0; // log2
-      while (across < 6 && (int64_t(word) << across) < nKeep)
-        ++across;
-      int64_t strips = ceilDiv(nKeep, int64_t(word) << across);
-      const bool words = nKeep >= word && strips <= int64_t(kMaxTickets);
-      if (!words)
-        strips = ceilDiv(nKeep, 256);
-      // (three blocks a CU stream best, measured in us at 256 / 384 / 768 /
-      // 1024 blocks: [5003, 3001] float64 41 / 35 / 34 / 36, [16384, 8192]
-      // float32 96 / 96 / 94 / 118; few strips leave the last blocks many
-      // chunks to fold: [16384, 16] float32 18.9 / 20.7 / 22.4 / 22.5)
-      const int64_t most = tuning().colsBlocks ? tuning().colsBlocks
-                           : !words            ? 2048
-                           : strips < 8        ? 256
-                                               : 768;
-      int64_t chunks = words ? most / strips : ceilDiv(most, strips);
-      if (chunks > nRed / 32)
-        chunks = nRed / 32;
-      if (chunks < 1)
-        chunks = 1;
-      if (chunks > 65535)
-        chunks = 65535;
-      const int64_t rowsPerChunk = ceilDiv(nRed, chunks);
-      chunks = ceilDiv(nRed, rowsPerChunk);
-      const Arg shape = Arg::I32(words ? across + 1 : 0);
-      void *partial =
-          chunks > 1 ? c->scratchFor(size_t(chunks) * size_t(nKeep) * accSize) : nullptr;
-      c->launch("nmk_reducecols_" + opAndType, size_t(strips), size_t(chunks), 1, 256, 1, 1,
-                {Arg::Ptr(x), Arg::Ptr(words || !partial ? out : partial), Arg::I64(nRed),
-                 Arg::I64(nKeep), Arg::I64(sr), Arg::I64(rowsPerChunk), shape,
-                 Arg::Ptr(partial), Arg::Ptr(c->tickets)});
-      if (partial && !words)
-        c->launch("nmk_reducecols_" + opAndAcc, size_t(ceilDiv(nKeep, 256)), 1, 1, 256, 1, 1,
-                  {Arg::Ptr(partial), Arg::Ptr(out), Arg::I64(chunks), Arg::I64(nKeep),
-                   Arg::I64(nKeep), Arg::I64(chunks), Arg::I32(0), Arg::Ptr(nullptr),
-                   Arg::Ptr(nullptr)});
-      return;
-    }
-    // A long contiguous run reduced to one value: a wave per chunk, then the
-    // chunks' results by one wave.
-    if (nKeep == 1 && sr == 1 && nRed >= 65536) {
-      // one block a chunk: as many as stream well at once, 16 KiB or more each
-      int64_t nChunks = ceilDiv(nRed * int64_t(16 / word), 16384);
-      const int64_t most = tuning().reduceBlocks ? tuning().reduceBlocks : 512;
-      if (nChunks > most)
-        nChunks = most;
-      // (chunks of whole 128-bit words, so that every chunk of an aligned
-      // array starts on one)
-      const int64_t chunk = ceilDiv(ceilDiv(nRed, nChunks), word) * word;
-      nChunks = ceilDiv(nRed, chunk);
-      void *partial = c->scratchFor(size_t(nChunks) * accSize);
-      c->launch("nmk_reducechunks_" + opAndType, size_t(nChunks), 1, 1, 256, 1, 1,
-                {Arg::Ptr(x), Arg::Ptr(partial), Arg::I64(nRed), Arg::I64(chunk),
-                 Arg::I64(nChunks), Arg::I32(aligned16(x) ? 1 : 0)});
-      c->launch("nmk_reduce_" + opAndAcc, 1, 1, 1, 256, 1, 1,
-                {Arg::Ptr(partial), Arg::Ptr(out), Arg::I64(1), Arg::I64(nChunks),
-                 Arg::I64(0), Arg::I64(1), Arg::I64(1), Arg::I32(0)});
-      return;
-    }
-    // Many short runs (the rows of a tall matrix of a few columns): a group
-    // of 1 to 32 lanes a kept index, two elements or so a lane.
-    if (nRed >= 1 && nRed <= 64 && nKeep >= 4096) {
-      int gShift = 0;
-      while (sr == 1 && (int64_t(2) << gShift) < nRed && gShift < 5)
-        ++gShift; // (a lane a kept index where the run is strided: the lanes then
-                  // follow the kept index, which has the shorter stride)
-      const int mode = 4 | (gShift << 8);
-      c->launchBlocksXY(std::string("nmk_reduce_") + opNames[op] + "_" + dtypeName(dtype),
-                        ceilDiv(nKeep << gShift, 256),
-                        {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(nKeep), Arg::I64(nRed),
-                         Arg::I64(sk), Arg::I64(sr), Arg::I64(1), Arg::I32(mode)});
-      return;
-    }
-    // (a block per kept index where the reduced run is long, a wave per
-    // kept index otherwise)
-    const bool wide = nRed >= 4096;
-    const int mode = ((sr == 1 && aligned16(x) && (nKeep == 1 || sk % word == 0)) ? 1 : 0) |
-                     (wide ? 2 : 0);
-    c->launchBlocksXY(std::string("nmk_reduce_") + opNames[op] + "_" + dtypeName(dtype),
-                      wide ? nKeep : ceilDiv(nKeep, 4),
-                      {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(nKeep), Arg::I64(nRed),
-                       Arg::I64(sk), Arg::I64(sr), Arg::I64(1), Arg::I32(mode)});
+NMHIP_EXPORT void nmhipReduceToHost(void *ctx, int op, int dtype, const void *x, int64_t n,
+                                    void *hostOut) {
+  guarded([&]() {
+    Context *c = toCtx(ctx);
+    std::lock_guard<std::mutex> lock(c->mutex);
+    const size_t bytes = dtype == NMHIP_F32 ? 4 : 8; // of the accumulator
+    c->resultToHost(hostOut, bytes, [&](void *out) {
+      reduceInto(c, op, dtype, x, 1, n, n, 1, -1, out);
+    });
   });
 }
 
@@ -976,19 +1025,16 @@ NMHIP_EXPORT void nmhipNorm2F32(void *ctx, const float *x, int64_t n,
   guarded([&]() {
     Context *c = toCtx(ctx);
     std::lock_guard<std::mutex> lock(c->mutex);
-    if (n < 0)
-      fail("nmhipNorm2F32: negative extent");
-    int64_t blocks = tuning().reduceBlocks ? tuning().reduceBlocks : kFullSumBlocks;
-    int64_t need = ceilDiv(n, 256 * 16);
-    if (need < 1)
-      need = 1;
-    if (blocks > need)
-      blocks = need;
-    void *partial = c->scratchFor(size_t(blocks) * 4);
-    c->launch("nmk_norm2_f32", size_t(blocks), 1, 1, 256, 1, 1,
-              {Arg::Ptr(x), Arg::Ptr(out), Arg::I64(n),
-               Arg::I32(aligned16(x) ? 1 : 0), Arg::Ptr(partial),
-               Arg::Ptr(c->tickets)});
+    norm2Into(c, x, n, out);
+  });
+}
+
+NMHIP_EXPORT void nmhipNorm2F32ToHost(void *ctx, const float *x, int64_t n, float *hostOut) {
+  guarded([&]() {
+    Context *c = toCtx(ctx);
+    std::lock_guard<std::mutex> lock(c->mutex);
+    c->resultToHost(hostOut, sizeof(float),
+                    [&](void *out) { norm2Into(c, x, n, static_cast<float *>(out)); });
   });
 }
 

@@ -688,9 +688,7 @@ class Dispatcher:
                             prod.left.id == prod.right.id:
                         x = array(prod.left)
                         if x is not None and x.dtype == np.float32:
-                            return self._served(
-                                "library", ops.sqrt_sum_squares(x).asnumpy().reshape(-1)[0],
-                                x.ctx)
+                            return self._served("library", ops.norm(x), x.ctx)
         except (TypeError, ValueError, NotImplementedError):
             return NotImplemented       # outside what the kernel covers: fuse instead
         return NotImplemented

@@ -44,13 +44,10 @@ class Context:
         self.handle = lib.nmhipContextCreate(device.encode() if device else None)
         self._finalizer = weakref.finalize(self, lib.nmhipContextDestroy,
                                            self.handle)
+        self.queue = lib.nmhipContextQueue(self.handle)
         # events of launches enqueued from Python and not yet retired, oldest
         # first (kernel_impl.LaunchPlan.enqueue / retire)
         self.pending = []
-
-    @property
-    def queue(self):
-        return lib.nmhipContextQueue(self.handle)
 
     def set_async(self, flag):
         lib.nmhipContextSetAsync(self.handle, 1 if flag else 0)
@@ -122,10 +119,10 @@ class _Buffer:
 class HipNdArray:
     def __init__(self, buffer, shape, dtype, strides, offset):
         self._buffer = buffer
-        self.shape = tuple(int(s) for s in shape)
+        self.shape = tuple(map(int, shape))
         self.dtype = np.dtype(dtype)
-        self.strides = tuple(int(s) for s in strides)  # bytes, as NumPy
-        self._offset = int(offset)                      # bytes
+        self.strides = tuple(map(int, strides))  # bytes, as NumPy
+        self._offset = int(offset)               # bytes
 
     # -- construction --------------------------------------------------------
     @classmethod
@@ -134,7 +131,7 @@ class HipNdArray:
             shape = (shape,)
         dtype = np.dtype(dtype)
         ctx = get_context(device)
-        count = int(np.prod(shape, dtype=np.int64)) if len(shape) else 1
+        count = math.prod(int(n) for n in shape)
         buf = _Buffer(ctx, count * dtype.itemsize, usm_type)
         return cls(buf, shape, dtype, _dense_strides(shape, dtype.itemsize, order),
                    0)
@@ -181,7 +178,8 @@ class HipNdArray:
 
     @property
     def elem_strides(self):
-        return tuple(s // self.dtype.itemsize for s in self.strides)
+        itemsize = self.dtype.itemsize
+        return tuple([s // itemsize for s in self.strides])
 
     @property
     def T(self):
@@ -265,10 +263,10 @@ class HipNdArray:
         }
 
     def is_c_contiguous(self):
-        if self.size == 0:
+        if 0 in self.shape:
             return True
         expect = self.dtype.itemsize
-        for n, s in zip(reversed(self.shape), reversed(self.strides)):
+        for n, s in zip(self.shape[::-1], self.strides[::-1]):
             if n != 1 and s != expect:
                 return False
             expect *= n
@@ -360,6 +358,8 @@ def empty(shape, dtype, usm_type="device", device=None):
 def disjoint(arrays):
     """True when no two of the device arrays share a byte (then the kernel may
     reorder their loads and stores freely)."""
+    if len({id(a._buffer) for a in arrays}) == len(arrays):
+        return True                       # an allocation each
     spans = []
     for a in arrays:
         lo = hi = a.ptr

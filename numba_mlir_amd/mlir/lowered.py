@@ -39,7 +39,9 @@ _SIGNATURES = {
                                     ctypes.c_int]),
     "nmhipReduce": (None, [_vp, ctypes.c_int, ctypes.c_int, _vp, _i64, _i64, _i64,
                            _i64, ctypes.c_int, _vp]),
+    "nmhipReduceToHost": (None, [_vp, ctypes.c_int, ctypes.c_int, _vp, _i64, _vp]),
     "nmhipNorm2F32": (None, [_vp, _vp, _i64, _vp]),
+    "nmhipNorm2F32ToHost": (None, [_vp, _vp, _i64, _vp]),
     "nmhipNorm2RowsF32": (None, [_vp, _vp, _i64, _i64, _i64, _vp]),
     "nmhipGemm": (None, [_vp, ctypes.c_int, _vp, _i64x2, _vp, _i64x2, _vp, _i64x2,
                          _i64, _i64, _i64, ctypes.c_double, ctypes.c_double]),

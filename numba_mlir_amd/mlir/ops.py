@@ -21,6 +21,15 @@ _DTYPES = {
 }
 
 
+# what a reduction of each type accumulates in
+_ACCUMULATORS = {
+    lowered.I32: lowered.ctypes.c_int64,
+    lowered.I64: lowered.ctypes.c_int64,
+    lowered.F32: lowered.ctypes.c_float,
+    lowered.F64: lowered.ctypes.c_double,
+}
+
+
 def _code(dtype):
     try:
         return _DTYPES[np.dtype(dtype)]
@@ -29,7 +38,7 @@ def _code(dtype):
 
 
 def _i64x2(a, b):
-    return (lowered.ctypes.c_int64 * 2)(int(a), int(b))
+    return lowered._i64x2(int(a), int(b))
 
 
 def _as_2d(arr, shape2):
@@ -50,24 +59,39 @@ def _as_2d(arr, shape2):
     return out
 
 
+def _broadcast(a, b):
+    """numpy.broadcast_shapes of two shapes (NumPy's own builds an array of
+    each: 4 us)."""
+    if len(a) < len(b):
+        a, b = b, a
+    shape = list(a)
+    for dim, n in enumerate(b, len(a) - len(b)):
+        if shape[dim] == 1:
+            shape[dim] = n
+        elif n != 1 and n != shape[dim]:
+            raise ValueError("shape mismatch: objects cannot be broadcast to a single shape: "
+                             f"{a} and {b}")
+    return tuple(shape)
+
+
 def _binary(op, a, b, out=None):
     a, b = asarray(a), asarray(b)
     if a.ndim > 2 or b.ndim > 2:
         raise NotImplementedError("maps are implemented for rank <= 2")
     # numpy.add etc.: operands are converted to the promoted dtype before the
     # generic (linalg_builder.py:297-305, broadcast_type 261-275).
-    dtype = np.promote_types(a.dtype, b.dtype)
-    if a.dtype != dtype or b.dtype != dtype:
+    dtype = a.dtype
+    if b.dtype != dtype:
         raise NotImplementedError("mixed-dtype maps need a convert kernel")
-    res_shape = np.broadcast_shapes(a.shape, b.shape)
+    res_shape = a.shape if a.shape == b.shape else _broadcast(a.shape, b.shape)
     if out is None:
         out = empty(res_shape, dtype, usm_type=a.usm_type, device=a.ctx.device)
     elif out.shape != tuple(res_shape) or out.dtype != dtype:
         raise ValueError("out has the wrong shape or dtype")
     shape2 = (1,) * (2 - len(res_shape)) + tuple(res_shape)
-    sa, sb, so = _as_2d(a, shape2), _as_2d(b, shape2), _as_2d(out, shape2)
-    # A size-1 output dimension still needs its real stride: recompute.
-    so = list((0,) * (2 - out.ndim) + out.elem_strides)
+    sa, sb = _as_2d(a, shape2), _as_2d(b, shape2)
+    # (a size-1 output dimension keeps its real stride)
+    so = (0,) * (2 - out.ndim) + out.elem_strides
     lib.nmhipMapBinary(a.ctx.handle, op, _code(dtype), a.ptr, _i64x2(*sa), b.ptr,
                        _i64x2(*sb), out.ptr, _i64x2(*so), shape2[0], shape2[1])
     return out
@@ -135,17 +159,18 @@ def _reduce(op, x, axis, result_dtype=None):
     # Integer reductions accumulate and return int64 (promote_int,
     # numpy/funcs.py:120-123, 176, 210); a full reduction is cast back to the
     # input dtype (185).
-    is_int = np.issubdtype(x.dtype, np.integer)
+    is_int = x.dtype.kind in "iu"
     acc_dtype = np.dtype(np.int64) if is_int else x.dtype
     n0, n1 = x2.shape
     s0, s1 = x2.elem_strides
     if axis is None:
-        out = empty((1,), acc_dtype, usm_type="device", device=x.ctx.device)
         if not x2.is_c_contiguous():
             raise NotImplementedError("full reduction needs a contiguous array")
-        lib.nmhipReduce(x.ctx.handle, op, _code(x.dtype), x2.ptr, n0, n1,
-                        n1, 1, -1, out.ptr)
-        res = out.asnumpy()[0]
+        code = _code(x.dtype)
+        out = _ACCUMULATORS[code]()
+        lib.nmhipReduceToHost(x.ctx.handle, op, code, x2.ptr, n0 * n1,
+                              lowered.ctypes.byref(out))
+        res = acc_dtype.type(out.value)
         return x.dtype.type(res) if result_dtype is None else result_dtype(res)
     out = empty((n1 if axis == 0 else n0,), acc_dtype, usm_type=x.usm_type,
                 device=x.ctx.device)
@@ -181,6 +206,16 @@ def sqrt_sum_squares(x, out=None):
         out = empty((1,), np.float32, usm_type="device", device=x.ctx.device)
     lib.nmhipNorm2F32(x.ctx.handle, x.ptr, x.size, out.ptr)
     return out
+
+
+def norm(x):
+    """``np.sqrt(np.sum(x * x))`` of a contiguous float32 array as a scalar."""
+    x = asarray(x)
+    if x.dtype != np.float32 or not x.is_c_contiguous():
+        raise ValueError("norm needs a contiguous float32 array")
+    out = lowered.ctypes.c_float()
+    lib.nmhipNorm2F32ToHost(x.ctx.handle, x.ptr, x.size, lowered.ctypes.byref(out))
+    return np.float32(out.value)
 
 
 def l2_norm_rows(a, out=None):
