@@ -1247,26 +1247,36 @@ gemm_thin_fold(const T *__restrict__ part, int slices, int m, int64_t C, int64_t
 // of every row filled with zeros, followed by rows of zeros up to Rp rows.
 // For operands whose rows do not begin or end on a word (an odd extent or
 // leading dimension, a view that starts inside a word), and to pad operands
-// to whole tiles.  One thread per destination word.
+// to whole tiles.  One thread per destination word; both operands of a product
+// in one launch (float32, us with a launch each / with one: 1800 x 1700 x 3001
+// 165.0 / 162.6, 2047 x 2049 x 2051 159.9 / 157.2).
+template <typename T> struct PackJob {
+  const T *src = nullptr;
+  int64_t ld = 0, R = 0, C = 0;
+  T *dst = nullptr;
+  int64_t Cp = 0, Rp = 0;
+  __host__ __device__ int64_t words() const { return Rp * (Cp / Mfma<T>::VEC); }
+  __host__ __device__ int64_t blocks() const { return (words() + 255) / 256; }
+};
 template <typename T>
-__global__ __launch_bounds__(256) void
-gemm_pack_rows(const T *__restrict__ src, int64_t ld, int64_t R, int64_t C,
-               T *__restrict__ dst, int64_t Cp, int64_t Rp) {
+__global__ __launch_bounds__(256) void gemm_pack_rows(PackJob<T> first, PackJob<T> second) {
   typedef typename Mfma<T>::Vec Vec;
   constexpr int VEC = Mfma<T>::VEC;
-  const int64_t wordsPerRow = Cp / VEC;
-  const int64_t word = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (word >= Rp * wordsPerRow)
+  const int64_t ahead = first.blocks();
+  const bool two = blockIdx.x >= ahead;
+  const PackJob<T> job = two ? second : first;
+  const int64_t word = (blockIdx.x - (two ? ahead : 0)) * 256 + threadIdx.x;
+  if (word >= job.words())
     return;
   int64_t r, c;
-  splitWord(word, wordsPerRow, r, c);
+  splitWord(word, job.Cp / VEC, r, c);
   c *= VEC;
-  const T *row = src + r * ld;
+  const T *row = job.src + r * job.ld;
   Vec v;
 #pragma unroll
   for (int q = 0; q < VEC; ++q)
-    v[q] = (r < R && c + q < C) ? row[c + q] : T(0);
-  *reinterpret_cast<Vec *>(dst + r * Cp + c) = v;
+    v[q] = (r < job.R && c + q < job.C) ? row[c + q] : T(0);
+  *reinterpret_cast<Vec *>(job.dst + r * job.Cp + c) = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -1650,6 +1660,19 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
                          ldz, alpha, beta);
   };
 
+  auto packBoth = [&](const PackJob<T> &first, const PackJob<T> &second) {
+    auto pack = [&](const PackJob<T> &a, const PackJob<T> &b) {
+      hipLaunchKernelGGL(gemm_pack_rows<T>, dim3(unsigned(a.blocks() + b.blocks())), dim3(256),
+                         0, stream, a, b);
+    };
+    if (first.blocks() + second.blocks() < int64_t(1) << 24) {
+      pack(first, second);
+    } else { // (more work-items than one launch counts)
+      pack(first, PackJob<T>());
+      pack(second, PackJob<T>());
+    }
+  };
+
   lastPacked = false;
   if (M > 0 && N > 0) {
     bool launched = false;
@@ -1989,14 +2012,19 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       // copies with only their stores guarded.  float32 4000^3: 117 -> 126
       // TFLOP/s, 4094^3: 117 -> 131; float64 4000^3: 56 -> 62, 7000 x 7500 x
       // 8000: 61 -> 65.  From 192 padded tiles on in float32 (below that the
-      // guarded 128 x 128 tiles in even shares are as fast or faster, 3000^3:
-      // 107 against 104), from 256 in float64 (the same tile either way: the
+      // guarded 128 x 128 tiles in even shares are as fast or faster, 2000 x
+      // 2300 x 2600: 175 us against 183), from 64 where an operand off the
+      // word grid is copied anyway (2047^3 143 -> 136 us, 2501^3 243 -> 225,
+      // 3001 x 2999 x 1001 166 -> 159; 36 tiles, 1500^3: 80 -> 100), from 256
+      // in float64 (the same tile either way: the
       // copies have to be won back from the guards on the loads alone).
       bool paddedBig = false, tilesInside = false;
       {
         constexpr int PT = sizeof(T) == 4 ? 256 : 128;
         const int64_t padSlots = sizeof(T) == 4 ? cus : slots;
-        const int64_t minTiles = sizeof(T) == 4 ? 3 * cus / 4 : cus;
+        const int64_t minTiles = sizeof(T) == 8   ? cus
+                                 : packX || packY ? cus / 4
+                                                  : 3 * cus / 4;
         auto roundUp = [](int64_t v, int64_t to) { return (v + to - 1) / to * to; };
         const int64_t Mp = roundUp(Mz, PT), Np = roundUp(Nz, PT), Kp = roundUp(K, BK);
         const bool fitsAsIs = Mz == Mp && Nz == Np && K % BK == 0 && !offWords(X, ldx, xC) &&
@@ -2031,15 +2059,8 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
             base = static_cast<unsigned char *>(heapWorkspace(device, packBytes));
           }
           if (base) {
-            auto pack = [&](const T *src, int64_t ld, int64_t R, int64_t C, int64_t Rp,
-                            int64_t Cp, T *dst) {
-              const int64_t words = Rp * (Cp / VEC);
-              hipLaunchKernelGGL(gemm_pack_rows<T>, dim3(unsigned((words + 255) / 256)),
-                                 dim3(256), 0, stream, src, ld, R, C, dst, Cp, Rp);
-            };
             T *Xp = reinterpret_cast<T *>(base), *Yp = reinterpret_cast<T *>(base + xBytes);
-            pack(X, ldx, xR, xC, xRp, xCp, Xp);
-            pack(Y, ldy, yR, yC, yRp, yCp, Yp);
+            packBoth({X, ldx, xR, xC, Xp, xCp, xRp}, {Y, ldy, yR, yC, Yp, yCp, yRp});
             const EvenShares even = sharesOf(evenBlocks, slabs, padTiles, Np / PT);
             dim3 grid(unsigned(Np / PT), unsigned(Mp / PT), 1);
             if (evenBlocks)
@@ -2115,21 +2136,17 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
           // was: the copies still fit, as checked above)
           unsigned char *base = W ? reinterpret_cast<unsigned char *>(W) - packBytes
                                   : static_cast<unsigned char *>(heapWorkspace(device, packBytes));
-          auto pack = [&](const T *src, int64_t ld, int64_t R, int64_t C, int64_t Cp, T *dst) {
-            const int64_t words = R * (Cp / VEC);
-            hipLaunchKernelGGL(gemm_pack_rows<T>, dim3(unsigned((words + 255) / 256)),
-                               dim3(256), 0, stream, src, ld, R, C, dst, Cp, R);
-          };
-          if (packX) {
-            T *dst = reinterpret_cast<T *>(base);
-            pack(X, ldx, xR, xC, xCp, dst);
-            X = dst;
-          }
-          if (packY) {
-            T *dst = reinterpret_cast<T *>(base + xBytes);
-            pack(Y, ldy, yR, yC, yCp, dst);
-            Y = dst;
-          }
+          T *Xp = reinterpret_cast<T *>(base), *Yp = reinterpret_cast<T *>(base + xBytes);
+          PackJob<T> jobX, jobY;
+          if (packX)
+            jobX = {X, ldx, xR, xC, Xp, xCp, xR};
+          if (packY)
+            jobY = {Y, ldy, yR, yC, Yp, yCp, yR};
+          packBoth(jobX, jobY);
+          if (packX)
+            X = Xp;
+          if (packY)
+            Y = Yp;
         }
         const int64_t ldxk = packX ? xCp : ldx, ldyk = packY ? yCp : ldy;
         const EvenShares even = sharesOf(evenBlocks, slabs, tilesM * tilesN, tilesN);
