@@ -1425,20 +1425,17 @@ SplitPlan planSplit(int64_t tiles, int64_t K, int BK, int64_t slots /* resident 
 }
 
 // Blocks of an even-shares launch over `tiles` block tiles of `slabs` K slabs
-// each on `slots` resident blocks, perCu of them a CU, or 0 when whole tiles do
-// as well: they fill their rounds to nine tenths or more, or a block's share
-// would be under eight slabs (the pieces' trip through the workspace would
-// cost more than the idle CUs).  Where two blocks share a CU, one that is
-// left alone there in the last round runs nearly twice as fast: whole tiles
-// in shares / as they are, us: 7000 x 7500 x 8000 float64, rounds filled to
-// 0.905, 12150 / 12061.  One block a CU gains up to a fill of 0.95 (8000 x
-// 7500 x 7000 float32, 0.94: 3972 / 4080; measured to four rounds).
-int planEvenShares(int64_t tiles, int64_t slabs, int64_t slots, int perCu) {
+// each on `slots` resident blocks, or 0 when whole tiles do as well: they
+// fill their rounds to nine tenths or more, or a block's share would be under
+// eight slabs (the pieces' trip through the workspace would cost more than
+// the idle CUs).  Above nine tenths it depends on K (in shares / whole, us:
+// float32 8000 x 7500 x 7000, 0.94 full, 3972 / 4080; 5632 x 8192 x 1024,
+// 0.92, 503 / 457; float64 7000 x 7500 x 8000, 0.905, 12150 / 12061).
+int planEvenShares(int64_t tiles, int64_t slabs, int64_t slots) {
   if (tiles <= 0 || slabs <= 0)
     return 0;
   const int64_t rounds = (tiles + slots - 1) / slots;
-  const int64_t enough = perCu == 1 && rounds <= 4 ? 95 : 90;
-  if (tiles * 100 >= rounds * slots * enough)
+  if (tiles * 10 >= rounds * slots * 9)
     return 0;
   if (tiles * slabs < 8 * slots)
     return 0;
@@ -1952,7 +1949,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       const bool bigFits = sizeof(T) == 4 && Mt % 256 == 0 && Nt % 256 == 0;
       const int64_t bigTiles = (Mt / 256) * (Nt / 256);
       const int bigEven = bigFits && workspaceKind == WORKSPACE_HEAP
-                              ? planEvenShares(bigTiles, Kt / BK, cus, 1)
+                              ? planEvenShares(bigTiles, Kt / BK, cus)
                               : 0;
       // (from 64 large tiles on: below, the 128 x 128 tiles in slices or
       // shares are as fast or faster -- 1792^3 120 against 131 us, 1024 x
@@ -2039,7 +2036,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
         tilesInside = sizeof(T) == 8 && wordsAligned && padTiles >= minTiles && Mz >= 128 &&
                       Nz >= 128 && (padTiles * 2 < 3 * cus || padTiles > 4 * cus);
         const int slabs = int(Kp / BK);
-        int evenBlocks = planEvenShares(padTiles, slabs, padSlots, int(padSlots / cus));
+        int evenBlocks = planEvenShares(padTiles, slabs, padSlots);
         if (!launched && canPack && !fitsAsIs && !tilesInside && (!whole || packX || packY) &&
             K >= 256 && padTiles >= minTiles &&
             Mp / PT <= 65535 && Mz <= 0x7fffffff - 256 &&
@@ -2119,7 +2116,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
         bool slicesFill = false;
         SplitPlan plan = planSlices(tilesM * tilesN, K, slicesFill);
         int evenBlocks = workspaceKind == WORKSPACE_HEAP && !slicesFill
-                             ? planEvenShares(tilesM * tilesN, slabs, slots, 2)
+                             ? planEvenShares(tilesM * tilesN, slabs, slots)
                              : 0;
         T *W = evenWorkspace(evenBlocks, 128, 128);
         if (evenBlocks)
@@ -2204,7 +2201,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
           plan = planSlices((Mt / BM) * (Nt / BN), Kt, slicesFill);
         int evenBlocks = big ? bigEven
                          : workspaceKind == WORKSPACE_HEAP && !slicesFill
-                             ? planEvenShares((Mt / BM) * (Nt / BN), slabs, slots, 2)
+                             ? planEvenShares((Mt / BM) * (Nt / BN), slabs, slots)
                              : 0;
         T *W = evenWorkspace(evenBlocks, BM, BN);
         if (evenBlocks)
