@@ -16,13 +16,20 @@
 // at K = 4096, 3.4e-7 against 4.1e-7 at 512; data in [0, 1): 5.3e-7 against
 // 8.5e-7 and 2.4e-7 against 3.1e-7).
 //
-// Which operands this holds for: every part must be a bf16 number.  A nonzero
-// |x| below 2^-100 could have parts below bf16's smallest, and an infinity, a
-// NaN or a value that rounds to infinity has none; a block that meets one
-// computes its piece of the result again with the float32 instructions, whose
-// results such inputs then have as before.  (A small one is seen by an integer
-// minimum over the operands, the others by what they leave in the
-// accumulators: a NaN.)
+// Which operands this holds for: every part must be a bf16 number and every
+// sum a float32.  Operands are multiplied by 2^23 on their way to LDS, and sums
+// by 2^-46 on their way out: the last bit of any float32, 2^-149 at least, then
+// lies in bf16's normal range, so values of any smallness have parts.  An
+// infinity, a NaN, an operand of 2^105 or a sum of 2^82 and more leaves a NaN
+// or an infinity in the accumulators.  They are looked at after 4 slabs, every
+// 64 and at the end; the 32 x 32 tiles that hold one are computed again with
+// the float32 instructions, whose results such inputs then have as before (at
+// once, if they are most of a wave's).  us at 4096^3, float32 instructions
+// alone / values of 2^-100 and less and all infinities computed again in whole
+// 256 x 256 tiles / this: exp(-x) for x in [0, 100) 980 / 1385 / 633, an infinity
+// in the last column of every 128th row 978 / 1832 / 1077, every sum too large
+// 980 / 1350 / 1153 (ordinary data 979 / 630 / 629); at 1024^3 45 / 68 / 41.5,
+// 45 / 64 / 55.5, 44.5 / 64 / 55.5.
 //
 // Time: six bf16 products take 6/16 of the float32 instructions' time.  At
 // 4096^3 the 256 x 256 tile takes 577 us (238 TFLOP/s of float32 product)
@@ -44,20 +51,7 @@ typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 
-// The smallest nonzero |x| of the values seen, as 2 |bits| - 1 (zero becomes
-// the largest number): 1.5 instructions a value.
-struct SmallestSeen {
-  uint32_t least = 0xffffffffu;
-  __device__ __forceinline__ void see(float x, float y) {
-    const uint32_t u = (__builtin_bit_cast(uint32_t, x) << 1) - 1u;
-    const uint32_t v = (__builtin_bit_cast(uint32_t, y) << 1) - 1u;
-    const uint32_t w = u < v ? u : v;
-    least = w < least ? w : least;
-  }
-  __device__ __forceinline__ bool tooSmall() const { // below 2^-100
-    return least < (uint32_t(127 - 100) << 24) - 1u;
-  }
-};
+constexpr float kPartsScale = 8388608.0f; // 2^23
 
 // The parts of two values, each pair packed into a register (nearest-even
 // conversions; the differences are exact).
@@ -136,12 +130,8 @@ template <int X, bool K_CONTIG, int THREADS> struct PartsFetch {
       p += 16 * ld;
     }
   }
-  // The next slab, of which `left` of K are left (1 or more).
+  // The next slab, of which `left` of K are left (1 to 15): the last one.
   __device__ __forceinline__ void fetchTail(int left) {
-    if (left >= 16) {
-      fetch();
-      return;
-    }
     if (K_CONTIG) {
 #pragma unroll
       for (int i = 0; i < NQ; ++i) {
@@ -162,6 +152,20 @@ template <int X, bool K_CONTIG, int THREADS> struct PartsFetch {
   }
 };
 
+// Both operands' next slab, of which `left` of K are left: one branch for the
+// two (where the ways of loading a whole and a cut slab meet, the second
+// operand's loads waited for the first's).
+template <typename FetchA, typename FetchB>
+__device__ __forceinline__ void fetchBoth(FetchA &fa, FetchB &fb, int left) {
+  if (left >= 16) {
+    fa.fetch();
+    fb.fetch();
+  } else {
+    fa.fetchTail(left);
+    fb.fetchTail(left);
+  }
+}
+
 // An operand's slab in LDS, in words of 16 bytes: three planes (h, m, l) of two
 // halves of K of X rows of eight bf16.  One word of padding a half: the halves
 // start 16 bytes apart among the banks.
@@ -171,14 +175,12 @@ template <int X> struct PartsSlab {
 
 template <int X, bool KC, int THREADS>
 __device__ __forceinline__ void stashParts(const PartsFetch<X, KC, THREADS> &f, uintx4 *lds,
-                                           SmallestSeen &seen) {
+                                           float scale) {
 #pragma unroll
   for (int i = 0; i < f.NQ; ++i) {
     uint32_t h0, h1, m0, m1, l0, l1;
-    seen.see(f.at(i, 0), f.at(i, 1));
-    seen.see(f.at(i, 2), f.at(i, 3));
-    partsOf(f.at(i, 0), f.at(i, 1), h0, m0, l0);
-    partsOf(f.at(i, 2), f.at(i, 3), h1, m1, l1);
+    partsOf(scale * f.at(i, 0), scale * f.at(i, 1), h0, m0, l0);
+    partsOf(scale * f.at(i, 2), scale * f.at(i, 3), h1, m1, l1);
     uintx2 *at = reinterpret_cast<uintx2 *>(lds) +
                  2 * (f.quad / 2 * PartsSlab<X>::HALF + f.rowOf(i)) + f.quad % 2;
     at[0] = uintx2{h0, h1};
@@ -274,7 +276,6 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
     PartsFetch<BN, !B_NC, THREADS> fb;
     fa.init(A, lda, bm, M, slab0 * BK, tid);
     fb.init(B, ldb, bn, N, slab0 * BK, tid);
-    SmallestSeen seen;
     floatx16 acc[TM][TN];
     auto clear = [&] {
 #pragma unroll
@@ -287,13 +288,11 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
     };
     clear();
 
-    fa.fetchTail(K - slab0 * BK);
-    fb.fetchTail(K - slab0 * BK);
-    stashParts(fa, As[0], seen);
-    stashParts(fb, Bs[0], seen);
+    fetchBoth(fa, fb, K - slab0 * BK);
+    stashParts(fa, As[0], kPartsScale);
+    stashParts(fb, Bs[0], kPartsScale);
     if (slab0 + 1 < slab1) {
-      fa.fetchTail(K - (slab0 + 1) * BK);
-      fb.fetchTail(K - (slab0 + 1) * BK);
+      fetchBoth(fa, fb, K - (slab0 + 1) * BK);
     }
     __syncthreads();
 
@@ -316,15 +315,14 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
       rowsOf(0);
       rowsOf(1);
       if (STASH) {
-        stashParts(fa, As[cur ^ 1], seen);
-        stashParts(fb, Bs[cur ^ 1], seen);
+        stashParts(fa, As[cur ^ 1], kPartsScale);
+        stashParts(fb, Bs[cur ^ 1], kPartsScale);
       }
       if (FETCH == 1) {
         fa.fetch();
         fb.fetch();
       } else if (FETCH == 2) {
-        fa.fetchTail(K - (s + 2) * BK);
-        fb.fetchTail(K - (s + 2) * BK);
+        fetchBoth(fa, fb, K - (s + 2) * BK);
       }
       constexpr int LEFT[6] = {2, 0, 1, 1, 0, 0}, RIGHT[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
@@ -344,70 +342,94 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
     typedef std::integral_constant<int, 0> No;
     typedef std::integral_constant<int, 1> Yes;
     typedef std::integral_constant<int, 2> Last;
-    bool again = false; // whether an operand had no parts
+    // The wave's 32 x 32 tiles, one bit each, that hold an infinity or a NaN.
+    auto tilesLost = [&] {
+      uint32_t lost = 0;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          float finite = 0.0f;
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            finite = __builtin_fmaf(acc[i][j][r], 0.0f, finite);
+          if (__builtin_amdgcn_ballot_w64(finite != finite))
+            lost |= 1u << (i * TN + j);
+        }
+      return lost;
+    };
+    uint32_t lost = 0;
     int s = slab0;
-    while (s + 3 < slab1 && !again) {
-      // (looked at every 64 slabs, so that such operands cost little more
-      // than the float32 instructions alone)
-      const int stop = s + 64 < slab1 - 3 ? s + 64 : slab1 - 3;
+    bool early = false; // given up before the end of K
+    for (int look = 4; s + 3 < slab1 && !early; look = 64) {
+      const int stop = s + look < slab1 - 3 ? s + look : slab1 - 3;
       for (; s < stop; ++s)
         slab(s, Yes(), Yes());
       if (stop < slab1 - 3)
-        again = __syncthreads_or(seen.tooSmall());
+        early = __syncthreads_or(2 * __builtin_popcount(tilesLost()) > TM * TN);
     }
-    if (!again) {
+    if (early) {
+      lost = (1u << (TM * TN)) - 1;
+    } else {
       if (s + 2 < slab1)
         slab(s++, Yes(), Last());
       if (s + 1 < slab1)
         slab(s++, Yes(), No());
       slab(s, No(), No());
-      float finite = 0.0f;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            finite = __builtin_fmaf(acc[i][j][r], 0.0f, finite);
-      again = __syncthreads_or(seen.tooSmall() || finite != finite);
+      lost = tilesLost();
     }
-    if (again) {
-      // The same piece with v_mfma_f32_32x32x2_f32: lane half h of the wave
-      // takes k = 8 h + t of the slab in step t.
-      clear();
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const float unscale = 1.0f / (kPartsScale * kPartsScale);
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          acc[i][j][r] = lost >> (i * TN + j) & 1 ? 0.0f : acc[i][j][r] * unscale;
+      }
+    if (__syncthreads_or(lost != 0)) {
+      // The lost tiles with v_mfma_f32_32x32x2_f32: lane half h of the wave
+      // takes k = 8 h + t of the slab in step t.  Two LDS stages, the next
+      // slab loaded while one is multiplied, one barrier a slab.
       fa.init(A, lda, bm, M, slab0 * BK, tid);
       fb.init(B, ldb, bn, N, slab0 * BK, tid);
+      fetchBoth(fa, fb, K - slab0 * BK);
 #pragma nounroll
       for (s = slab0; s < slab1; ++s) {
-        fa.fetchTail(K - s * BK);
-        fb.fetchTail(K - s * BK);
-        __syncthreads(); // every wave has read the last slab
-        stashFloats(fa, As[0]);
-        stashFloats(fb, Bs[0]);
-        __syncthreads();
-        floatx4 b[TN][2];
+        const int cur = (s - slab0) & 1;
+        stashFloats(fa, As[cur]);
+        stashFloats(fb, Bs[cur]);
+        __syncthreads(); // (also: every wave has read the slab before the last)
+        if (s + 1 < slab1)
+          fetchBoth(fa, fb, K - (s + 1) * BK);
+        floatx4 a[TM][2], b[TN][2];
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+        for (int w = 0; w < 2; ++w) {
 #pragma unroll
-          for (int w = 0; w < 2; ++w)
-            b[j][w] = reinterpret_cast<const floatx4 *>(Bs[0])[2 * (bWord + j * 32) + w];
+          for (int j = 0; j < TN; ++j)
+            b[j][w] = reinterpret_cast<const floatx4 *>(Bs[cur])[2 * (bWord + j * 32) + w];
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+            a[i][w] = reinterpret_cast<const floatx4 *>(As[cur])[2 * (aWord + i * 32) + w];
+        }
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int w = 0; w < 2; ++w) {
-            const floatx4 a = reinterpret_cast<const floatx4 *>(As[0])[2 * (aWord + i * 32) + w];
+          for (int j = 0; j < TN; ++j)
+            if (lost >> (i * TN + j) & 1)
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-              for (int j = 0; j < TN; ++j)
-                acc[i][j] =
-                    __builtin_amdgcn_mfma_f32_32x32x2f32(a[t], b[j][w][t], acc[i][j], 0, 0, 0);
-          }
+              for (int t = 0; t < 8; ++t)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                    a[i][t / 4][t % 4], b[j][t / 4][t % 4], acc[i][j], 0, 0, 0);
       }
     }
 
     // A whole tile goes to C, scaled; a piece of one goes to its workspace
     // slot as a dense BM x BN block, unscaled.
+    // (The lane's number as if it were new, so that the places in C are worked
+    // out here: the compiler would keep them in scratch over the whole of K.)
+    int home = lane;
+    asm volatile("" : "+v"(home));
     float *out = C + int64_t(bm) * ldc + bn;
     int64_t ldo = ldc;
     float scale = alpha, keep = beta;
@@ -424,10 +446,10 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const int col = wn * (TN * 32) + j * 32 + lane % 32;
+        const int col = wn * (TN * 32) + j * 32 + home % 32;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int row = wm * (TM * 32) + i * 32 + Mfma<float>::accRow(r, lane);
+          const int row = wm * (TM * 32) + i * 32 + Mfma<float>::accRow(r, home);
           if (!(row < rowsLeft && col < colsLeft))
             continue;
           float *dst = out + int64_t(row) * ldo + col;
