@@ -105,3 +105,20 @@ def test_large_results(env, m, n, k):
     for ea, eb in ((50, 50), (60, 55), (110, -20), (120, -100), (30, 63)):
         got = _product(hip, ops, np.ldexp(a0, ea), np.ldexp(b0, eb)).astype(np.float64)
         assert (np.abs(np.ldexp(got, -ea - eb) - truth) <= bound).all()
+
+
+@pytest.mark.parametrize("m,n", [(640, 768), (2048, 2047), (4096, 4096)])
+def test_one_and_two_products(env, m, n):
+    """K = 1: every product rounded to nearest.  K = 2: one rounding of a product
+    and one of the sum."""
+    hip, ops = env
+    rng = np.random.default_rng(m)
+    for draw in (rng.standard_normal, rng.random):
+        a = draw((m, 2)).astype(np.float32)
+        b = draw((2, n)).astype(np.float32)
+        got = _product(hip, ops, np.ascontiguousarray(a[:, :1]), np.ascontiguousarray(b[:1]))
+        assert np.array_equal(got, a[:, :1] * b[:1])
+        truth = a.astype(np.float64) @ b.astype(np.float64)
+        larger = np.maximum(np.abs(a[:, :1] * b[:1]), np.abs(a[:, 1:] * b[1:]))
+        bound = 2.0 ** -24 * (larger + np.abs(truth)) * 1.000001
+        assert (np.abs(_product(hip, ops, a, b) - truth) <= bound).all()
