@@ -8,13 +8,23 @@
 // is then the sum of nine exact bf16 products, of which
 //   h l' + l h' + m m' + m h' + h m' + h h'
 // are computed, smallest first, and the other three left out: together they
-// are below 2^-24 |x y|, less than the rounding of one float32 product.  The
-// matrix core adds the sixteen products of an instruction to a float32
-// accumulator, so a sum over K is rounded 6 K / 16 times instead of K times:
-// against float64 the results are closer than the float32 instructions' (2-norm
-// of the error over 2-norm of the result, normal data: 1.0e-6 against 1.15e-6
-// at K = 4096, 3.4e-7 against 4.1e-7 at 512; data in [0, 1): 5.3e-7 against
-// 8.5e-7 and 2.4e-7 against 3.1e-7).
+// are below 2^-24 |x y|, less than the rounding of one float32 product.  An
+// instruction adds its sixteen products to a float32 accumulator in two groups
+// of eight (measured, element by element): within a group what lies below 2^-24
+// of the largest term is cut off, downwards, then the sum is rounded to nearest.
+// A sum over K is so rounded 12 K / 16 times at most, and six of those count,
+// instead of K times.  The cut leans every sum the same way: accumulators and
+// A's parts change sign after 32 slabs and then every 64, and from one slice or
+// piece of K to the next, so that what one leaned another takes back.
+//
+// 2-norm of the error against float64 over 2-norm of the result, float32
+// instructions / this, centred data: K = 3 3.6e-8 / 3.3e-8, 16 7.4e-8 / 3.4e-8, 512
+// 2.1e-7 / 1.7e-7, 4096 1.15e-6 / 0.98e-6, 16384 2.29e-6 / 1.88e-6, 262144 (in
+// slices) 2.29e-6 / 1.89e-6 (without the changes of sign 2.08e-6 at 16384,
+// 3.71e-6 at 262144); data in [0, 1): 4096 8.4e-7 / 5.2e-7, 16384 1.68e-6 /
+// 1.03e-6, 262144 4.3e-7 / 2.6e-7 (4.5e-7).  A sum of which one or two products
+// are not zero (a diagonal matrix times another) is not the nearest float32 as
+// the float32 instructions' is, but within 1.7e-7 of itself.
 //
 // Which operands this holds for: every part must be a bf16 number and every
 // sum a float32.  Operands are multiplied by 2^23 on their way to LDS, and sums
@@ -294,9 +304,16 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
     // 3.6e-8, 3.3e-8): they stay with the float32 instructions (and with the
     // small tile: the large one's shapes begin at K = 16).
     bool early = BM == 128 && K <= 2; // the parts are given up before the end of K
+    // A's scale, and its sign the accumulators': it changes from slice to slice
+    // and from piece to piece of a tile, and along a longer K.
+    // (The bits of it, so that it stays in a scalar register.)
+    uint32_t turned = ((sliceK > 0 ? blockIdx.z : piece ? blockIdx.x : 0) & 1) << 31;
+    auto left = [&] {
+      return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, kPartsScale) ^ turned);
+    };
     if (!early) {
       fetchBoth(fa, fb, K - slab0 * BK);
-      stashParts(fa, As[0], kPartsScale);
+      stashParts(fa, As[0], left());
       stashParts(fb, Bs[0], kPartsScale);
       if (slab0 + 1 < slab1)
         fetchBoth(fa, fb, K - (slab0 + 1) * BK);
@@ -322,7 +339,7 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
       rowsOf(0);
       rowsOf(1);
       if (STASH) {
-        stashParts(fa, As[cur ^ 1], kPartsScale);
+        stashParts(fa, As[cur ^ 1], left());
         stashParts(fb, Bs[cur ^ 1], kPartsScale);
       }
       if (FETCH == 1) {
@@ -367,12 +384,27 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
     };
     uint32_t lost = 0;
     int s = slab0;
-    for (int look = 4; s + 3 < slab1 && !early; look = 64) {
+    for (int look = 4; s + 3 < slab1 && !early; look = look == 4 ? 28 : 64) {
       const int stop = s + look < slab1 - 3 ? s + look : slab1 - 3;
-      for (; s < stop; ++s)
+      const bool more = stop < slab1 - 3;
+      const bool turn = more && look > 4;
+      for (; s < (turn ? stop - 1 : stop); ++s)
         slab(s, Yes(), Yes());
-      if (stop < slab1 - 3)
+      if (turn) {
+        turned ^= 1u << 31; // of slab `stop`, which is split now
+        slab(s++, Yes(), Yes());
+      }
+      if (more) {
         early = __syncthreads_or(2 * __builtin_popcount(tilesLost()) > TM * TN);
+        const float sign = turn ? -1.0f : 1.0f;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+              acc[i][j][r] *= sign;
+      }
     }
     if (early) {
       lost = (1u << (TM * TN)) - 1;
@@ -388,10 +420,12 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const float unscale = 1.0f / (kPartsScale * kPartsScale);
+        const float unscale = 1.0f / (left() * kPartsScale);
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          acc[i][j][r] = lost >> (i * TN + j) & 1 ? 0.0f : acc[i][j][r] * unscale;
+          acc[i][j][r] = lost >> (i * TN + j) & 1
+                             ? 0.0f
+                             : __builtin_fmaf(acc[i][j][r], unscale, 0.0f); // (no -0)
       }
     if (__syncthreads_or(lost != 0)) {
       // The lost tiles with v_mfma_f32_32x32x2_f32: lane half h of the wave
@@ -448,34 +482,39 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
       rowsLeft = BM;
       colsLeft = BN;
     }
-    auto store = [&](auto bare) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int col = wn * (TN * 32) + j * 32 + home % 32;
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int row = wm * (TM * 32) + i * 32 + Mfma<float>::accRow(r, home);
-            if (!decltype(bare)::value && !(row < rowsLeft && col < colsLeft))
-              continue;
-            float *dst = out + int64_t(row) * ldo + col;
-            float v = scale * acc[i][j][r];
-            if (!decltype(bare)::value && keep != 0.0f)
-              v += keep * *dst;
-            *dst = v;
-          }
-        }
-      }
-    };
     // (bare stores where nothing is cut off or added: the guarded ones are five
     // times the instructions, which a product of a slab or two waits for: 1024 x
     // 1024 x 16 21.9 -> 20.0 us, 640 x 640 x 64 23.8 -> 22.0.  The large tile's
     // products hide them, and it has no registers for both.)
-    if (BM == 128 && keep == 0.0f && rowsLeft >= BM && colsLeft >= BN)
-      store(std::true_type());
-    else
-      store(std::false_type());
+    const bool bare = BM == 128 && keep == 0.0f && rowsLeft >= BM && colsLeft >= BN;
+    if (bare) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            out[int64_t(wm * (TM * 32) + i * 32 + Mfma<float>::accRow(r, home)) * ldo +
+                wn * (TN * 32) + j * 32 + home % 32] = scale * acc[i][j][r];
+    }
+#pragma unroll
+    for (int i = 0; i < TM && !bare; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int col = wn * (TN * 32) + j * 32 + home % 32;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int row = wm * (TM * 32) + i * 32 + Mfma<float>::accRow(r, home);
+          if (!(row < rowsLeft && col < colsLeft))
+            continue;
+          float *dst = out + int64_t(row) * ldo + col;
+          float v = scale * acc[i][j][r];
+          if (keep != 0.0f)
+            v += keep * *dst;
+          *dst = v;
+        }
+      }
+    }
   } // segments
 }
 
