@@ -480,10 +480,10 @@ __device__ __forceinline__ ACC foldInPairs(ACC (&v)[N], Op op) {
 // Bound by memory: [5003, 3001] int32 column sums (60 MB) take 16.1 us, in two
 // launches of one element a lane 21.7.
 //
-// words == 0 (rows shorter than a word, or more strips than tickets): a block
-// owns 256 consecutive kept indices, one a lane, eight loads in flight;
-// several chunks leave their results at out[chunk * nKeep + k], and the same
-// kernel folds them.
+// words == 0 (rows shorter than a word, or odd ones of more strips than there
+// are tickets): a block owns 256 consecutive kept indices, one a lane, eight
+// loads in flight; several chunks leave their results at out[chunk * nKeep + k],
+// and the same kernel folds them.
 template <typename IN, typename ACC, typename Op>
 __device__ __forceinline__ void
 reduceColumns(const IN *__restrict__ x, ACC *__restrict__ out, int64_t nRed,

@@ -881,7 +881,14 @@ void reduceInto(Context *c, int op, int dtype, const void *x, int64_t n0, int64_
     while (across < 6 && (int64_t(word) << across) < nKeep)
       ++across;
     int64_t strips = ceilDiv(nKeep, int64_t(word) << across);
-    const bool words = nKeep >= word && strips <= int64_t(kMaxTickets);
+    // More strips than tickets fill the GPU in one chunk, which draws none.
+    // Words win there where every row begins and ends on one, us by elements /
+    // by words: [200, 1048832] float32 161 / 143, [200, 600000] float64 187 / 163,
+    // [64, 2000000] float32 103 / 96; not across the lines of odd rows: [200,
+    // 2000001] float32 282 / 290, [200, 2000002] int32 289 / 305.
+    const bool wholeWords = aligned16(x) && sr % word == 0 && nKeep % word == 0;
+    const bool words =
+        nKeep >= word && (strips <= int64_t(kMaxTickets) || wholeWords);
     if (!words)
       strips = ceilDiv(nKeep, 256);
     // (three blocks a CU stream best, measured in us at 256 / 384 / 768 /
@@ -895,7 +902,7 @@ void reduceInto(Context *c, int op, int dtype, const void *x, int64_t n0, int64_
     int64_t chunks = words ? most / strips : ceilDiv(most, strips);
     if (chunks > nRed / 32)
       chunks = nRed / 32;
-    if (chunks < 1)
+    if (chunks < 1 || (words && strips > int64_t(kMaxTickets)))
       chunks = 1;
     if (chunks > 65535)
       chunks = 65535;

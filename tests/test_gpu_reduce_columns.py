@@ -63,3 +63,16 @@ def test_nans_lose_and_infinities_pass(hip, dtype):
     odd = ~np.isfinite(want)
     assert np.array_equal(sums[odd], want[odd], equal_nan=True)
     assert np.isfinite(sums[~odd]).all()
+
+
+@pytest.mark.parametrize("dtype,cols", [(np.float32, 1048577 + 256), (np.float32, 1048580),
+                                        (np.int32, 1048844), (np.float64, 524418)])
+def test_more_strips_than_tickets(hip, dtype, cols):
+    """Over 4096 strips of columns, in one chunk: words of rows that are whole
+    ones, elements of others."""
+    from numba_mlir_amd.mlir import ops
+    x = np.random.default_rng(cols).integers(-9, 9, (70, cols), endpoint=True).astype(dtype)
+    d = hip.asarray(x)
+    assert np.array_equal(ops.sum(d, axis=0).asnumpy(), x.sum(axis=0))
+    assert np.array_equal(ops.amin(d, axis=0).asnumpy(), x.min(axis=0))
+    assert np.array_equal(ops.amax(d[:, 1:], axis=0).asnumpy(), x[:, 1:].max(axis=0))
