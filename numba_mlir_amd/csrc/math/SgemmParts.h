@@ -452,15 +452,24 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
           for (int i = 0; i < TM; ++i)
             a[i][w] = reinterpret_cast<const floatx4 *>(As[cur])[2 * (aWord + i * 32) + w];
         }
+        auto multiply = [&](int i, int j, int t) {
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][t / 4][t % 4], b[j][t / 4][t % 4],
+                                                           acc[i][j], 0, 0, 0);
+        };
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j)
-            if (lost >> (i * TN + j) & 1)
+          for (int j = 0; j < TN; ++j) {
+            if (!(lost >> (i * TN + j) & 1))
+              continue;
+            multiply(i, j, 0);
+            multiply(i, j, 1);
+            if (BM == 128 && K <= 2)
+              continue; // (the other steps multiply zeros: 1 us)
 #pragma unroll
-              for (int t = 0; t < 8; ++t)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                    a[i][t / 4][t % 4], b[j][t / 4][t % 4], acc[i][j], 0, 0, 0);
+            for (int t = 2; t < 8; ++t)
+              multiply(i, j, t);
+          }
       }
     }
 
