@@ -18,6 +18,8 @@
 #include <cstdlib>
 #include <mutex>
 
+#include "PackJobs.h"
+
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -1250,21 +1252,14 @@ gemm_thin_fold(const T *__restrict__ part, int slices, int m, int64_t C, int64_t
 // to whole tiles.  One thread per destination word; both operands of a product
 // in one launch (float32, us with a launch each / with one: 1800 x 1700 x 3001
 // 165.0 / 162.6, 2047 x 2049 x 2051 159.9 / 157.2).
-template <typename T> struct PackJob {
-  const T *src = nullptr;
-  int64_t ld = 0, R = 0, C = 0;
-  T *dst = nullptr;
-  int64_t Cp = 0, Rp = 0;
-  __host__ __device__ int64_t words() const { return Rp * (Cp / Mfma<T>::VEC); }
-  __host__ __device__ int64_t blocks() const { return (words() + 255) / 256; }
-};
+template <typename T> using PackJobOf = PackJob<T, Mfma<T>::VEC>;
 template <typename T>
-__global__ __launch_bounds__(256) void gemm_pack_rows(PackJob<T> first, PackJob<T> second) {
+__global__ __launch_bounds__(256) void gemm_pack_rows(PackJobOf<T> first, PackJobOf<T> second) {
   typedef typename Mfma<T>::Vec Vec;
   constexpr int VEC = Mfma<T>::VEC;
   const int64_t ahead = first.blocks();
   const bool two = blockIdx.x >= ahead;
-  const PackJob<T> job = two ? second : first;
+  const PackJobOf<T> job = two ? second : first;
   const int64_t word = (blockIdx.x - (two ? ahead : 0)) * 256 + threadIdx.x;
   if (word >= job.words())
     return;
@@ -1657,17 +1652,13 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
                          ldz, alpha, beta);
   };
 
-  auto packBoth = [&](const PackJob<T> &first, const PackJob<T> &second) {
-    auto pack = [&](const PackJob<T> &a, const PackJob<T> &b) {
-      hipLaunchKernelGGL(gemm_pack_rows<T>, dim3(unsigned(a.blocks() + b.blocks())), dim3(256),
-                         0, stream, a, b);
-    };
-    if (first.blocks() + second.blocks() < int64_t(1) << 24) {
-      pack(first, second);
-    } else { // (more work-items than one launch counts)
-      pack(first, PackJob<T>());
-      pack(second, PackJob<T>());
-    }
+  auto packBoth = [&](const PackJobOf<T> &first, const PackJobOf<T> &second) {
+    launchPacks(first, second, (int64_t(1) << 24) - 1,
+                [&](const PackJobOf<T> &a, const PackJobOf<T> &b) {
+                  hipLaunchKernelGGL(gemm_pack_rows<T>,
+                                     dim3(unsigned(a.blocks() + b.blocks())), dim3(256), 0,
+                                     stream, a, b);
+                });
   };
 
   lastPacked = false;
@@ -2134,7 +2125,7 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
           unsigned char *base = W ? reinterpret_cast<unsigned char *>(W) - packBytes
                                   : static_cast<unsigned char *>(heapWorkspace(device, packBytes));
           T *Xp = reinterpret_cast<T *>(base), *Yp = reinterpret_cast<T *>(base + xBytes);
-          PackJob<T> jobX, jobY;
+          PackJobOf<T> jobX, jobY;
           if (packX)
             jobX = {X, ldx, xR, xC, Xp, xCp, xR};
           if (packY)
