@@ -104,6 +104,9 @@ def _dense_strides(shape, itemsize, order="C"):
     return tuple(strides)
 
 
+_MOST_BYTES = 2 ** 63 - 1    # sizes and extents are 64-bit integers below Python
+
+
 class _Buffer:
     """Owner of one gpuxAlloc allocation."""
 
@@ -130,9 +133,11 @@ class HipNdArray:
         if isinstance(shape, int):
             shape = (shape,)
         dtype = np.dtype(dtype)
-        ctx = get_context(device)
-        count = math.prod(int(n) for n in shape)
-        buf = _Buffer(ctx, count * dtype.itemsize, usm_type)
+        extents = [int(n) for n in shape]
+        nbytes = math.prod(extents) * dtype.itemsize
+        if nbytes > _MOST_BYTES or (nbytes == 0 and extents and max(extents) > _MOST_BYTES):
+            raise OverflowError(f"an array of shape {tuple(extents)} is too large")
+        buf = _Buffer(get_context(device), nbytes, usm_type)
         return cls(buf, shape, dtype, _dense_strides(shape, dtype.itemsize, order),
                    0)
 
