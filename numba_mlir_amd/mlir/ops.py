@@ -81,7 +81,8 @@ def _binary(op, a, b, out=None):
     # numpy.add etc.: operands are converted to the promoted dtype before the
     # generic (linalg_builder.py:297-305, broadcast_type 261-275).
     dtype = a.dtype
-    if b.dtype != dtype:
+    if b.dtype != dtype or not dtype.isnative:
+        np.promote_types(dtype, b.dtype)    # (TypeError where no type holds both)
         raise NotImplementedError("mixed-dtype maps need a convert kernel")
     res_shape = a.shape if a.shape == b.shape else _broadcast(a.shape, b.shape)
     if out is None:

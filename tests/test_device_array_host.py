@@ -1,6 +1,8 @@
 """Host-only checks of the device array front: what it refuses before anything
 reaches a device."""
 
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -17,7 +19,8 @@ class _FakeBuffer:
 @pytest.fixture
 def no_device(monkeypatch):
     monkeypatch.setattr(device_array, "_Buffer", _FakeBuffer)
-    monkeypatch.setattr(device_array, "get_context", lambda device=None: None)
+    monkeypatch.setattr(device_array, "get_context",
+                        lambda device=None: SimpleNamespace(device=device, handle=None))
 
 
 @pytest.mark.parametrize("shape", [2 ** 70, (2 ** 64,), (3, 2 ** 63), (2 ** 70, 0), (2 ** 62, 8)])
@@ -32,3 +35,16 @@ def test_shapes_beyond_64_bits_are_refused(no_device, shape):
 def test_shapes_that_fit(no_device, shape, count):
     x = device_array.empty(shape, np.float64)
     assert x._buffer.nbytes == 8 * count and x.size == count
+
+
+@pytest.mark.parametrize("a,b,error", [
+    (">f4", ">f4", NotImplementedError),          # (promoted to the native type)
+    (">f4", "<f4", NotImplementedError),
+    (np.float32, np.float64, NotImplementedError),
+    (np.float32, "M8[s]", TypeError),             # no common type
+    (np.complex64, np.complex64, TypeError),      # no kernel
+])
+def test_maps_of_other_types_are_refused_as_before(no_device, a, b, error):
+    x, y = device_array.empty(4, a), device_array.empty(4, b)
+    with pytest.raises(error):
+        ops.add(x, y)
