@@ -2020,12 +2020,11 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
         const int64_t padTiles = (Mp / PT) * (Np / PT);
         // Operands on the word grid need no copies in float64 where tiles
         // can be moved inside them (GUARD 3), us with copies / without:
-        // 2000^3 305 / 278, 2400 x 2300 x 1000 235 / 224, 2500 x 2750 x 3000
-        // 722 / 683, 5000 x 5010 x 1000 889 / 867, 7000 x 7500 x 8000 12284 /
-        // 12087.  (From 1.5 to 4 tiles a CU the copies stay: the "+packed" of
-        // nmhipMathLastKernel is relied upon there.)
+        // 2000^3 305 / 278, 2500 x 2750 x 3000 714 / 677, 2040 x 4090 x 600
+        // 177 / 167, 4000 x 4000 x 1000 517 / 498, 7000 x 7500 x 8000 12284 /
+        // 12087 (from 1.5 to 4 tiles a CU, twelve shapes in four layouts: 2 to 8 %).
         tilesInside = sizeof(T) == 8 && wordsAligned && padTiles >= minTiles && Mz >= 128 &&
-                      Nz >= 128 && (padTiles * 2 < 3 * cus || padTiles > 4 * cus);
+                      Nz >= 128;
         const int slabs = int(Kp / BK);
         int evenBlocks = planEvenShares(padTiles, slabs, padSlots);
         if (!launched && canPack && !fitsAsIs && !tilesInside && (!whole || packX || packY) &&

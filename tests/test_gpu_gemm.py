@@ -721,9 +721,12 @@ def test_split_k_beta_zero_ignores_c(env):
     (np.float64, 1024, 1024, 4096, "dgemm_mfma_128x128_splitk"),
     (np.float64, 1000, 1100, 1200, "dgemm_mfma_128x128_ragged_splitk"),  # the reference's preset
     (np.float32, 1152, 1152, 1152, "sgemm_mfma_128x128_splitk"),
-    # float64 from 256 padded tiles on: the same tile over zero-padded copies
-    (np.float64, 2500, 2750, 3000, "dgemm_mfma_128x128_even+packed"),
-    (np.float64, 2040, 4090, 600, "dgemm_mfma_128x128+packed"),
+    # float64 tiles moved inside the operands; off the word grid from 256 padded
+    # tiles on, the same tile over zero-padded copies
+    (np.float64, 2500, 2750, 3000, "dgemm_mfma_128x128_ragged_even"),
+    (np.float64, 2040, 4090, 600, "dgemm_mfma_128x128_ragged"),
+    (np.float64, 2501, 2751, 3001, "dgemm_mfma_128x128_even+packed"),
+    (np.float64, 2041, 4091, 601, "dgemm_mfma_128x128+packed"),
 ])
 @pytest.mark.parametrize("ta,tb,tc", [(False, False, False), (True, False, True),
                                       (False, True, False)])
