@@ -4,8 +4,8 @@
 // Entry points, argument meaning and layout rules follow the oneMKL-backed
 // runtime they replace (reference:
 // numba_mlir/numba_mlir/math_runtime/sycl/lib/NumpyLinalg.cpp:67-183); the
-// arithmetic is a hand-written LDS-tiled MFMA kernel for gfx950 (fp32 and
-// fp64 matrix cores) plus a strided fallback.
+// arithmetic is hand-written LDS-tiled MFMA kernels for gfx950 (float64 on its
+// matrix cores, float32 in bf16 parts: SgemmParts.h) plus a strided fallback.
 #include "numba_mlir_hip/GpuQueueInterface.hpp"
 #include "numba_mlir_hip/MathRuntime.h"
 
@@ -1458,8 +1458,8 @@ bool splitFills(const SplitPlan &plan, int64_t tiles, int64_t slots) {
   if (plan.slices < 2)
     return false;
   // (two or three slices leave shares few pieces to add up, so the slices
-  // must fill more: 225 tiles x 2 fill 0.88 and lose to shares, 149 against
-  // 141 us for 1920^3 float32)
+  // must fill more: 225 tiles x 2 fill 0.88 and lose to shares in float64, 260
+  // against 248 us for 1920^3; in float32, 108 against 112, they would not)
   const int64_t pct = plan.slices >= 4 ? 86 : 93;
   return tiles * plan.slices * 100 >= slots * pct || plan.slices >= 16;
 }
@@ -1606,10 +1606,10 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
   const int64_t slots = 2 * cus; // resident blocks of the 128 x 128 tiles: two a CU
   // Equal slices of K for `tiles` 128 x 128 tiles, and whether they go ahead
   // of even shares.  float64 blocks share a CU in pairs; float32 ones may
-  // (186 registers a lane), which pays where one block a CU would not fill
-  // the GPU but two do (72 tiles: 3 slices fill 0.84 of 256 blocks, 7 fill
-  // 0.98 of 512; 1000 x 1100 x 1200 58 -> 52 us, 1280^3 64 -> 59), and not
-  // otherwise (1024^3: 4 slices on 256 blocks 40 us, 8 on 512 43).  The
+  // (under 256 registers a lane), which pays where one block a CU would not
+  // fill the GPU but two do (72 tiles: 3 slices fill 0.84 of 256 blocks, 7 fill
+  // 0.98 of 512; us with one / two, 1000 x 1100 x 1200 50.5 / 47.0, 1280^3 58.6 /
+  // 52.7), and not otherwise (1024^3: 4 slices on 256 blocks 39.5, 8 on 512 41.8).  The
   // entry point that may not allocate keeps to 256 blocks: the fixed
   // workspace is sized for those.
   auto planSlices = [&](int64_t tiles, int64_t k, bool &fills) {
@@ -1761,8 +1761,8 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       // gemm_thin_rows when the long one has unit stride along k,
       // gemm_thin_cols when along its other dimension.
       if (!launched && K > 32) {
-        // (by columns up to 16 of them: 16 x 16384 x 16384 float32 701 us on the
-        // tiles, 372 here; by rows the thin operand's reads cost more than
+        // (by columns up to 16 of them: 16 x 16384 x 16384 float32 461 us on the
+        // tiles, 343 here; by rows the thin operand's reads cost more than
         // the tiles' idle rows beyond 8)
         constexpr int64_t kLong = 1024, kThinRows = 8, kThinCols = 16;
         auto wordsOk = [&](const T *S, int64_t ld) { return aligned16(S) && ld % VEC == 0; };
@@ -1926,11 +1926,10 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       }
       // The matrix-core kernel takes the part of the problem that is whole
       // tiles, Z[0:Mt, 0:Nt] over k in [0, Kt); the strided kernel adds the
-      // rest of K to that block and computes the rows and columns beyond it
-      // (4000^3: 3968 x 3968 x 4000 on the matrix cores, 26 -> 65 TFLOP/s).
+      // rest of K to that block and computes the rows and columns beyond it.
       // float32: 256 x 256 block tiles (one block per CU on a 4096^2
       // problem) when the shape allows and there are enough tiles to fill the
-      // 256 CUs, 128 x 128 otherwise (4096^3: 577 against 704 us; the larger
+      // 256 CUs, 128 x 128 otherwise (4096^3: 620 against 713 us; the larger
       // tile halves the operand traffic and the splitting into parts).
       // float64: 128 x 128.
       const int64_t Mt = Mz - Mz % 128, Nt = Nz - Nz % 128, Kt = K - K % BK;
@@ -1942,17 +1941,15 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       const int bigEven = bigFits && workspaceKind == WORKSPACE_HEAP
                               ? planEvenShares(bigTiles, Kt / BK, cus)
                               : 0;
-      // (from 64 large tiles on: below, the 128 x 128 tiles in slices or
-      // shares are as fast or faster -- 1792^3 120 against 131 us, 1024 x
-      // 1024 x 4096 92 against 99 -- and from 121 on the large tile wins,
-      // 3072^3 456 against 474)
+      // (from 64 large tiles on, us with the large / the small tiles: 1024 x
+      // 1024 x 4096, 16 large tiles, 81 / 74; 1792^3, 49, 105 / 97; 2048^3, 64,
+      // 119 / 121; 2560^3, 100, 204 / 216; 2816^3, 121, 256 / 252; 3072^3, 144,
+      // 313 / 340)
       // (the tile counts below are a quarter and three quarters of the CUs)
       bool big = bigFits && bigTiles * 4 >= cus && (bigEven > 0 || bigTiles * 4 >= 3 * cus);
       if (big && bigTiles * 4 < 3 * cus) {
         // (fewer large tiles than CUs only pay in even shares: without room
-        // for those, the 128 x 128 tiles take the shape.  Slices of K on the
-        // large tile were measured and gain nothing over its even shares:
-        // 2048^3 160 against 158 us.)
+        // for those, the 128 x 128 tiles take the shape)
         int blocks = bigEven;
         (void)evenWorkspace(blocks, 256, 256);
         big = blocks > 0;
@@ -1971,16 +1968,19 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       // operand's contiguous dimension a multiple of the word): one launch
       // of 128 x 128 tiles that read zeros beyond the operands and store
       // only inside Z.
-      const bool wordsWhole = (xKc ? K : Mz) % VEC == 0 && (yNc ? Nz : K) % VEC == 0;
       const int64_t tilesM = (Mz + 127) / 128, tilesN = (Nz + 127) / 128;
-      // (only K ragged: the tiles as they are plus the rest of K on the
-      // strided kernel is faster, 116 against 106 TFLOP/s on 4096 x 4096 x 4100)
+      // (only K ragged, in float64 below a tile a CU: the tiles as they are plus
+      // the rest of K on the strided kernel.  It reads and writes C once more and
+      // is the slower way since the tile kernels take the end of K themselves, us
+      // this way / all of K on the tiles: float32 2048 x 2048 x 2052 138 / 120,
+      // 1920 x 1920 x 1932 131 / 114, float64 2048 x 1536 x 518 115 / 99)
       const bool onlyK = Mt == Mz && Nt == Nz && mostly;
       // An operand whose rows do not begin and end on 128-bit words (an odd
       // extent or leading dimension, a base inside a word) is copied once
       // into word-aligned rows padded with zeros (gemm_pack_rows) and the same
       // guarded tiles run on the copy: reading and writing each operand once
-      // more is small beside the product (4094^3 float32: 27 -> 110 TFLOP/s).
+      // more is small beside the product (4094^3 float32: 181 TFLOP/s, 27 on the
+      // strided kernel).
       // Needs the heap workspace.
       const int64_t xC = xKc ? K : Mz, xR = xKc ? Mz : K; // X: contiguous extent, rows
       const int64_t yC = yNc ? Nz : K, yR = yNc ? K : Nz;
@@ -1992,20 +1992,18 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       const bool packY = canPack && offWords(Y, ldy, yC);
       const bool wordsOk = (packX || !offWords(X, ldx, xC)) && (packY || !offWords(Y, ldy, yC));
       const bool wordsAligned = !offWords(X, ldx, xC) && !offWords(Y, ldy, yC);
-      (void)wordsWhole;
       // Large shapes that are not whole tiles of whole words (256 x 256 for
       // float32, 128 x 128 for float64), where padding them to such tiles
       // costs under a tenth more arithmetic: both operands are copied into
       // zero-padded rows (whole tiles, whole K slabs) and the tiles run on the
-      // copies with only their stores guarded.  float32 4000^3: 117 -> 126
-      // TFLOP/s, 4094^3: 117 -> 131; float64 4000^3: 56 -> 62, 7000 x 7500 x
-      // 8000: 61 -> 65.  From 192 padded tiles on in float32 (below that the
-      // guarded 128 x 128 tiles in even shares are as fast or faster, 2000 x
-      // 2300 x 2600: 175 us against 183), from 64 where an operand off the
-      // word grid is copied anyway (2047^3 143 -> 136 us, 2501^3 243 -> 225,
-      // 3001 x 2999 x 1001 166 -> 159; 36 tiles, 1500^3: 80 -> 100), from 256
-      // in float64 (the same tile either way: the
-      // copies have to be won back from the guards on the loads alone).
+      // copies with only their stores guarded.  us on 128 x 128 tiles / on such
+      // copies: float32 4000^3 696 / 645, 4094^3 758 / 666, float64 off the word
+      // grid (moved tiles on copies of the rows alone) 4095 x 4097 x 4099 2176 /
+      // 2168, 2501 x 2751 x 3001 723 / 718, 6001 x 6003 x 1001 1165 / 1154.  From
+      // 192 padded tiles on in float32 (2000 x 2300 x 2600, 99, 167 / 176;
+      // 3000^3, 144, 337 / 333), from 64 where an operand off the word grid is
+      // copied anyway (2047^3 135 / 131, 2501^3 232 / 217, 3001 x 2999 x 1001
+      // 155 / 152; 36 tiles, 1501^3, 81 / 92), from 256 in float64.
       bool paddedBig = false, tilesInside = false;
       {
         constexpr int PT = sizeof(T) == 4 ? 256 : 128;
@@ -2091,7 +2089,8 @@ int deviceGemm(void *queueObj, const typename MemrefOf<T>::type *a,
       }
       // (fewer than 16 tiles go to the strided kernel's 32 x 32 tiles, unless
       // K is long and the result a quarter of a tile or more: slices of K fill
-      // the GPU then -- 300 x 65536 x 300 float32 15 -> 60 TFLOP/s)
+      // the GPU then -- 300 x 65536 x 300 float32 88 TFLOP/s, 15 on the strided
+      // kernel)
       if (paddedBig || launched) {
         // (done)
       } else if (((!whole && (!onlyK || tilesInside)) || packX || packY) && copiesFit && unitOk && wordsOk && K > 0 &&
