@@ -24,10 +24,12 @@ def _product(hip, ops, a, b, ta=False, tb=False):
 
 
 def _bound(k):
-    """|error| / (|a| |b|): three products left out, 2^-24 in all, and one
-    rounding (2^-23 at most, the matrix core truncates) of the accumulator for
-    each of the six instructions of 16 elements of K, one more for a slab that
-    is not whole and four for the pieces of a tile."""
+    """|error| / (|a| |b|): three products left out, 2^-24 in all, and for each of
+    the six instructions of 16 elements of K two roundings to nearest of the
+    accumulator, 2^-24 of it each (what an instruction cuts off besides is under
+    2^-24 of a product), six instructions more for a slab that is not whole and
+    four roundings of the pieces of a tile.  A bound for every element; it grows
+    too fast with K to see a part product missing: the 2-norm below does."""
     return 2.0 ** -24 + 2.0 ** -23 * (6 * (k / 16 + 1) + 4)
 
 
@@ -67,6 +69,57 @@ def test_no_less_accurate_than_a_sum_in_float32(env):
         assert np.linalg.norm(got - truth) <= np.linalg.norm(plain - truth)
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (640, 516, 200), (1024, 1024, 1040), (1500, 1496, 600),   # the 128 x 128 tile: whole, slices, shares
+    (4096, 3072, 512), (6144, 3072, 256),                     # the 256 x 256 tile
+    (2048, 2048, 1040), (2560, 2304, 2064),                   # its even shares
+    (4000, 4000, 530), (2501, 2499, 777),                     # padded copies
+])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+def test_two_norm_of_the_error(env, m, n, k, ta, tb):
+    """Every part product counts.  A rounding to nearest leaves 2.5e-8 of the
+    value (root mean square over its binade); the r-th of 12 k / 16 roundings is
+    of a sum of the variance r / (12 k / 16) of the result's, so their errors are
+    2.5e-8 sqrt(12 k / 32) of it, and the result's own rounding adds one.  A
+    tenth more allowed; h l' or m m' left out would be 2^-18 / 3 = 1.3e-6."""
+    hip, ops = env
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    b = rng.standard_normal((k, n), dtype=np.float32)
+    truth = a.astype(np.float64) @ b.astype(np.float64)
+    error = np.linalg.norm(_product(hip, ops, a, b, ta, tb) - truth) / np.linalg.norm(truth)
+    assert error <= 1.1 * 2.5e-8 * np.sqrt(1 + 12 * k / 32)
+
+
+@pytest.mark.parametrize("m,k", [(640, 516), (516, 1200), (4096, 3072), (2048, 2048), (2047, 2051)])
+@pytest.mark.parametrize("ta", [False, True])
+def test_every_bit_of_a_permuted_matrix(env, m, k, ta):
+    """A times a permutation with signs: all 24 bits of every value arrive."""
+    hip, ops = env
+    rng = np.random.default_rng(m)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    order, signs = rng.permutation(k), rng.choice([-1.0, 1.0], k).astype(np.float32)
+    b = np.zeros((k, k), np.float32)
+    b[order, np.arange(k)] = signs
+    assert np.array_equal(_product(hip, ops, a, b, ta), a[:, order] * signs)
+
+
+@pytest.mark.parametrize("m,n,k", [(640, 516, 64), (4096, 3072, 64), (2048, 2048, 272)])
+def test_products_near_the_smallest_float(env, m, n, k):
+    """Products and sums among the subnormal numbers: the bound of others, and
+    one rounding to a multiple of 2^-149 of the result or of each piece of it."""
+    hip, ops = env
+    rng = np.random.default_rng(k)
+    a0 = rng.standard_normal((m, k), dtype=np.float32)
+    b0 = rng.standard_normal((k, n), dtype=np.float32)
+    truth = a0.astype(np.float64) @ b0.astype(np.float64)
+    scale = np.abs(a0).astype(np.float64) @ np.abs(b0).astype(np.float64)
+    for ea, eb in ((-60, -62), (-66, -64), (-70, -66), (-90, -52)):
+        got = _product(hip, ops, np.ldexp(a0, ea), np.ldexp(b0, eb)).astype(np.float64)
+        error = np.abs(np.ldexp(got, -ea - eb) - truth)
+        assert (error <= _bound(k) * scale + 4 * 2.0 ** (-150 - ea - eb)).all()
+
+
 def test_whole_numbers_are_exact(env):
     """Products and sums below 2^24 are float32 numbers, and come out as they are."""
     hip, ops = env
@@ -83,8 +136,9 @@ def test_whole_numbers_are_exact(env):
 @pytest.mark.parametrize("m,n,k", [(640, 516, 1200), (3072, 4096, 1200), (2048, 2048, 1200)])
 @pytest.mark.parametrize("ta", [False, True])
 def test_operands_without_parts(env, m, n, k, ta):
-    """Infinities, NaNs, values that round to infinity in bf16 and values so
-    small that their parts would underflow: the float32 instructions' results."""
+    """Infinities, NaNs and values that round to infinity in bf16: the float32
+    instructions' results.  Values so small that parts of them as they are would
+    underflow: float32's accuracy."""
     hip, ops = env
     rng = np.random.default_rng(5)
     a0 = rng.standard_normal((m, k), dtype=np.float32)
