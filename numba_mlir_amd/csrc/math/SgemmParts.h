@@ -13,9 +13,9 @@
 // of eight (measured, element by element): within a group what lies below 2^-24
 // of the largest term is cut off, downwards, then the sum is rounded to nearest:
 // 12 roundings for 16 terms of K, where the float32 instructions round each of
-// the 16.  The cut leans every sum the same way: accumulators and
-// A's parts change sign after 32 slabs and then every 64, and from one slice or
-// piece of K to the next, so that what one leaned another takes back.
+// the 16.  The cut leans every sum the same way: accumulators and A's parts
+// change sign after 64 slabs and then every 128, and from one slice or piece of
+// K to the next, so that what one leaned another takes back.
 //
 // 2-norm of the error against float64 over 2-norm of the result, float32
 // instructions / this, centred data: K = 3 3.6e-8 / 3.3e-8, 16 7.4e-8 / 3.4e-8, 512
@@ -31,15 +31,15 @@
 // by 2^-46 on their way out: the last bit of any float32, 2^-149 at least, then
 // lies in bf16's normal range, so values of any smallness have parts.  An
 // infinity, a NaN, an operand of 2^105 or a sum of 2^82 and more leaves a NaN
-// or an infinity in the accumulators.  They are looked at after 4 slabs, every
-// 64 and at the end; the 32 x 32 tiles that hold one are computed again with
+// or an infinity in the accumulators.  They are looked at after 4, 64 and every
+// 128 slabs and at the end; the 32 x 32 tiles that hold one are computed again with
 // the float32 instructions, whose results such inputs then have as before (at
 // once, if they are most of a wave's).  us at 4096^3, float32 instructions
 // alone / values of 2^-100 and less and all infinities computed again in whole
-// 256 x 256 tiles / this: exp(-x) for x in [0, 100) 980 / 1385 / 633, an infinity
-// in the last column of every 128th row 978 / 1832 / 1077, every sum too large
-// 980 / 1350 / 1153 (ordinary data 979 / 630 / 629); at 1024^3 45 / 68 / 41.5,
-// 45 / 64 / 55.5, 44.5 / 64 / 55.5.
+// 256 x 256 tiles / this: exp(-x) for x in [0, 100) 970 / 1284 / 613, an infinity
+// in the last column of every 128th row 969 / 1715 / 1029, every sum too large
+// 969 / 1281 / 1144 (ordinary data 972 / 617 / 613); at 1024^3 44.3 / 67.0 / 38.6,
+// 44.4 / 63.0 / 47.9, 44.4 / 63.0 / 54.7.
 //
 // Time: six bf16 products take 6/16 of the float32 instructions' time.  At
 // 4096^3 the 256 x 256 tile takes 577 us (238 TFLOP/s of float32 product)
@@ -384,27 +384,28 @@ sgemm_parts(const float *__restrict__ A, const float *__restrict__ B, float *__r
     };
     uint32_t lost = 0;
     int s = slab0;
-    for (int look = 4; s + 3 < slab1 && !early; look = look == 4 ? 28 : 64) {
+    // (A look costs 0.7 us on the large tile, as a third of a slab.  Where the end
+    // is 24 slabs away or nearer there is none: 1000 x 1100 x 1200, of 11 slabs a
+    // slice, 48.1 us with one, 47.4 without; of all sums too large 55 / 57.)
+    for (int look = slab1 - slab0 > 24 ? 4 : 24; s + 3 < slab1 && !early;
+         look = look == 4 ? 60 : 128) {
       const int stop = s + look < slab1 - 3 ? s + look : slab1 - 3;
-      const bool more = stop < slab1 - 3;
-      const bool turn = more && look > 4;
+      const bool more = stop < slab1 - 3, turn = more && look > 4;
       for (; s < (turn ? stop - 1 : stop); ++s)
         slab(s, Yes(), Yes());
       if (turn) {
         turned ^= 1u << 31; // of slab `stop`, which is split now
         slab(s++, Yes(), Yes());
-      }
-      if (more) {
-        early = __syncthreads_or(2 * __builtin_popcount(tilesLost()) > TM * TN);
-        const float sign = turn ? -1.0f : 1.0f;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-              acc[i][j][r] *= sign;
+              acc[i][j][r] = -acc[i][j][r];
       }
+      if (more)
+        early = __syncthreads_or(2 * __builtin_popcount(tilesLost()) > TM * TN);
     }
     if (early) {
       lost = (1u << (TM * TN)) - 1;
