@@ -42,10 +42,10 @@
 // 44.4 / 63.0 / 47.9, 44.4 / 63.0 / 54.7.
 //
 // Time: six bf16 products take 6/16 of the float32 instructions' time.  At
-// 4096^3 the 256 x 256 tile takes 577 us (238 TFLOP/s of float32 product)
-// against 966 us; the matrix cores are busy 76 % of the cycles at 1.78 GHz,
-// the clock the power limit leaves (a loop of nothing but these instructions:
-// 96 % at 1.86 GHz).
+// 4096^3 the 256 x 256 tile takes 577 to 640 us by box and temperature (238 to
+// 215 TFLOP/s of float32 product) against 966 us; the matrix cores are busy 71
+// to 76 % of the cycles at 1.77 GHz, the clock the power limit leaves (a loop of
+// nothing but these instructions: 96 % at 1.86 GHz).
 #pragma once
 
 #include <hip/hip_runtime.h>
