@@ -92,12 +92,11 @@ void nmrtMathRuntimeFinalize(void);
  * tile kernel's name when the blocks took even shares of all K slabs, "_splitk" after
  * either when K was cut into slices, "<tile kernel>+edges" when the strided
  * kernel completed what the tiles left, "+packed" when an operand whose rows
- * do not begin and end on 128-bit words was first copied into padded rows);
- * for tests and profiling.  The name is that of the shape's plan: a product
- * whose 128 x 128 tiles would be few or short runs on tiles of 16 to 48 rows whose
- * waves share out K (gemm_fine, one launch, no copies) under the name its plan
- * on 128 x 128 tiles, or the strided kernel, has, and so does a float32 product
- * whose operands are split into parts ahead of it (sgemm_planes). */
+ * do not begin and end on 128-bit words was first copied into padded rows;
+ * "sgemm_fine", "dgemm_fine" for tiles of 16 to 48 rows whose waves share out K;
+ * "sgemm_planes" for operands split into their parts ahead of the tiles, "_even"
+ * behind it when the last of those went in shares of K); for tests and
+ * profiling. */
 const char *nmhipMathLastKernel(void);
 
 #ifdef __cplusplus

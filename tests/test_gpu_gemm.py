@@ -86,11 +86,20 @@ def test_internal_gemm_fixture_grid(env):
 
 
 @pytest.mark.parametrize("ta,tb,tc", list(itertools.product([False, True], repeat=3)))
-@pytest.mark.parametrize("m,n,k", [(33, 29, 47), (128, 128, 16), (1, 1, 1), (64, 1, 300),
-                                   (256, 384, 64), (4096, 3072, 32), (4096, 3072, 48),
-                                   (3072, 4096, 96), (300, 260, 100), (257, 129, 17),
-                                   (1000, 1000, 1000), (131, 4100, 40), (1500, 2000, 52)])
-def test_layouts_against_float64(env, ta, tb, tc, m, n, k):
+@pytest.mark.parametrize("m,n,k,kernel", [
+    # under 16 of K and few tiles: the strided kernel; else few or short tiles share out K
+    (1, 1, 1, "sgemm_generic"), (33, 29, 15, "sgemm_generic"), (300, 260, 15, "sgemm_generic"),
+    (257, 129, 13, "sgemm_generic"), (33, 29, 47, "sgemm_fine"), (64, 1, 300, "sgemm_fine"),
+    (256, 384, 64, "sgemm_fine"), (300, 260, 100, "sgemm_fine"), (257, 129, 17, "sgemm_fine"),
+    (131, 4100, 40, "sgemm_fine"),
+    # whole tiles
+    (128, 128, 16, "sgemm_mfma_128x128"), (4096, 3072, 32, "sgemm_mfma_256x256"),
+    (4096, 3072, 48, "sgemm_mfma_256x256"), (3072, 4096, 96, "sgemm_mfma_256x256"),
+    # tiles whose ends lie outside
+    (1000, 1000, 1000, "sgemm_mfma_128x128_ragged"), (1500, 2000, 52, "sgemm_mfma_128x128_ragged"),
+    (100, 4100, 20, "sgemm_mfma_128x128_ragged"),
+])
+def test_layouts_against_float64(env, ta, tb, tc, m, n, k, kernel):
     """Every stride pattern the entry point accepts (row/column major A, B, C)."""
     hip, ops, orc, mrt = env
     rng = np.random.default_rng(m * 1000 + n * 10 + k)
@@ -101,17 +110,7 @@ def test_layouts_against_float64(env, ta, tb, tc, m, n, k):
     d_c = _to_dev(hip, lay(c0, tc))
     ops.gemm(_to_dev(hip, lay(a, ta)), _to_dev(hip, lay(b, tb)), d_c, 0.5, 2.0)
     got = d_c.asnumpy()
-    mt, nt, kt = m - m % 128, n - n % 128, k - k % 16
-    if (mt, nt, kt) == (m, n, k):
-        # every layout of a tile-aligned problem runs on the matrix cores
-        assert _kernel(mrt) in ("sgemm_mfma_128x128", "sgemm_mfma_256x256")
-    elif -(-m // 128) * -(-n // 128) < 16:
-        assert mrt.last_kernel() == "sgemm_generic"
-    else:
-        # whole tiles on the matrix cores, the edges on the strided kernel
-        # (when the leading dimensions allow 128-bit loads)
-        assert _kernel(mrt) in ("sgemm_generic", "sgemm_mfma_128x128+edges",
-                                     "sgemm_mfma_256x256+edges", "sgemm_mfma_128x128_ragged")
+    assert _kernel(mrt) == kernel
     truth = 2.0 * c0 + 0.5 * (a.astype(np.float64) @ b.astype(np.float64))
     bound = 1e-5 * (2.0 * np.abs(c0) + 0.5 * (np.abs(a).astype(np.float64) @ np.abs(b))) + 1e-30
     assert (np.abs(got - truth) <= bound).all()
@@ -124,9 +123,11 @@ def _check_scaled(got, a, b, c0, alpha, beta, rel):
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
-@pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("m,n,k", [(2000, 1500, 1000), (1540, 1420, 2004), (1412, 1536, 20),
-                                   (4100, 4200, 36), (516, 520, 4)])
+@pytest.mark.parametrize("dtype,m,n,k", [
+    (np.float32, 1400, 1100, 1000), (np.float32, 1140, 1420, 2004), (np.float32, 2000, 1500, 4000),
+    (np.float64, 2000, 1500, 1000), (np.float64, 1540, 1420, 2004)] + [
+    (dtype, *shape) for dtype in (np.float32, np.float64)
+    for shape in ((1412, 1536, 20), (4100, 4200, 36), (516, 520, 4))])
 def test_ragged_shapes_on_tiles_that_read_zeros_outside(env, dtype, m, n, k, ta, tb):
     """Shapes that are not whole tiles but whose 128-bit words are whole run
     in one launch of tiles that read zeros beyond the operands and store only
@@ -165,7 +166,9 @@ def test_operands_off_the_word_grid_are_repacked(env, dtype):
     wider arrays, odd extents, a base inside a word) are copied once into
     word-aligned rows padded with zeros and run on the guarded tiles."""
     hip, ops, orc, mrt = env
-    m, n, k = 1540, 2052, 1001
+    single = dtype == np.float32
+    # (float32 from 148 tiles on: parts split ahead; float64 under 4e9 products: small tiles)
+    m, n, k = (1540, 1284, 1001) if single else (1540, 2052, 1301)
     rng = np.random.default_rng(5)
     a_wide = rng.standard_normal((m, k + 3)).astype(dtype)
     b = rng.standard_normal((k, n)).astype(dtype)
@@ -178,11 +181,11 @@ def test_operands_off_the_word_grid_are_repacked(env, dtype):
                   1e-5 if dtype == np.float32 else 1e-13)
     tol = 1e-5 if dtype == np.float32 else 1e-13
     lay = lambda x, t: np.asfortranarray(x) if t else x
-    for (m, n, k), ta, tb, tc in (((1001, 1003, 1005), False, False, False),
-                                  ((1001, 1003, 1005), True, False, True),
-                                  ((777, 1025, 2049), True, True, False),
-                                  ((513, 2047, 300), False, False, False),
-                                  ((2047, 2049, 2051), False, False, False)):
+    for (m, n, k), ta, tb, tc in (((1001, 1003, 1005 if single else 4005), False, False, False),
+                                  ((1001, 1003, 1005 if single else 4005), True, False, True),
+                                  ((777, 1025, 2049 if single else 5051), True, True, False),
+                                  ((513, 2047, 31 if single else 15), False, False, False),
+                                  ((2047, 2049, 4051 if single else 2051), False, False, False)):
         a = rng.standard_normal((m, k)).astype(dtype)
         b = rng.standard_normal((k, n)).astype(dtype)
         c0 = rng.standard_normal((m, n)).astype(dtype)
@@ -191,7 +194,7 @@ def test_operands_off_the_word_grid_are_repacked(env, dtype):
         assert mrt.last_kernel().endswith("+packed"), mrt.last_kernel()
         _check_scaled(d_c.asnumpy(), a, b, c0, 1.5, -0.5, tol)
     # whole tiles, but the first operand starts one element into a word
-    m = n = k = 1024
+    m, n, k = 1024, 1024, 4096
     a = rng.standard_normal((m, k)).astype(dtype)
     b = rng.standard_normal((k, n)).astype(dtype)
     flat = np.zeros(m * k + 1, dtype)
@@ -248,8 +251,8 @@ def _check(got, a, b):
     assert np.linalg.norm(got - truth) <= 1e-4 * np.linalg.norm(truth)
 
 
-@pytest.mark.parametrize("m,n,k", [(128, 128, 16), (256, 384, 512), (128, 256, 4096),
-                                   (1024, 1024, 1024), (384, 128, 48),
+@pytest.mark.parametrize("m,n,k", [(128, 128, 16), (256, 384, 4096), (128, 256, 4096),
+                                   (1024, 1024, 1024), (384, 128, 32),
                                    (4096, 3072, 64), (3584, 3584, 16)])
 def test_mfma_kernel(env, m, n, k):
     hip, ops, orc, mrt = env
@@ -580,12 +583,12 @@ def test_small_products_of_long_operands(env, dtype, k, m, n):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("m,k,n", [(16, 1 << 18, 16), (32, 100_003, 20), (100, 50_000, 60),
+@pytest.mark.parametrize("m,k,n", [(16, 1 << 18, 16), (32, 100_003, 20), (100, 200_000, 60),
                                    (128, 1 << 17, 128), (300, 1 << 15, 300), (10, 4099, 12)])
 def test_few_tiles_with_a_long_k(env, dtype, m, k, n):
-    """Results of a few tiles from long operands: K is cut into as many
-    slices as fill the GPU, on the strided kernel for the smallest results
-    and on the guarded tiles from a quarter of a tile on."""
+    """Results of a few tiles from long operands: K is cut into slices, on
+    the tiles of 16 to 48 rows for the smallest results and on the guarded tiles
+    from a quarter of a tile on."""
     hip, ops, _, mrt = env
     rng = np.random.default_rng(m + k + n)
     x = rng.standard_normal((k, m)).astype(dtype)
@@ -596,7 +599,7 @@ def test_few_tiles_with_a_long_k(env, dtype, m, k, n):
         d_c = hip.asarray(c0)
         ops.gemm(d_a, hip.asarray(b), d_c, 1.5, -0.5)
         assert "_splitk" in mrt.last_kernel(), mrt.last_kernel()
-        assert ("generic" in mrt.last_kernel()) == (m * n < 4096)
+        assert ("fine" in mrt.last_kernel()) == (m * n < 4096)
         _check_scaled(d_c.asnumpy(), a, b, c0, 1.5, -0.5, tol)
 
 
@@ -629,7 +632,7 @@ def test_identity_and_linearity_full_size(env):
 
 
 @pytest.mark.parametrize("ta,tb,tc", list(itertools.product([False, True], repeat=3)))
-@pytest.mark.parametrize("m,n,k", [(128, 128, 16), (256, 384, 80), (1024, 1024, 1024)])
+@pytest.mark.parametrize("m,n,k", [(128, 128, 16), (256, 384, 16), (1024, 1024, 4096)])
 def test_float64_mfma(env, ta, tb, tc, m, n, k):
     """mkl_gemm_float64_device on the fp64 matrix cores, every layout; the
     tolerance is rel 1e-5 (float64 bar), met with a wide margin."""
@@ -658,11 +661,14 @@ def test_float64_gemm(env):
 
 # ---- split K: few tiles, long K ------------------------------------------------
 
-@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("ta,tb,tc", [(False, False, False), (True, False, False),
                                       (False, True, True), (True, True, False)])
-@pytest.mark.parametrize("m,n,k", [(1024, 1024, 1024), (128, 256, 4096), (512, 384, 2000),
-                                   (1000, 1000, 1000), (640, 516, 1028), (1280, 1280, 272)])
+@pytest.mark.parametrize("dtype,m,n,k", [
+    (np.float32, 1024, 1024, 1024), (np.float32, 128, 256, 4096), (np.float32, 512, 384, 2000),
+    (np.float32, 1000, 1000, 1000), (np.float32, 640, 516, 1028), (np.float32, 1280, 1280, 1104),
+    # (float64 from 4e9 products on: under that tiles of 16 to 48 rows share out K)
+    (np.float64, 1024, 1024, 4096), (np.float64, 128, 256, 131072), (np.float64, 512, 384, 24000),
+    (np.float64, 1000, 1000, 4100), (np.float64, 640, 516, 12200), (np.float64, 1280, 1280, 2448)])
 def test_split_k(env, dtype, ta, tb, tc, m, n, k):
     """Shapes with too few tiles to fill the GPU cut K into slices whose
     partial products are added in slice order: every layout, alpha and beta
@@ -687,9 +693,9 @@ def test_split_k(env, dtype, ta, tb, tc, m, n, k):
 
 def test_split_k_beta_zero_ignores_c(env):
     hip, ops, _, mrt = env
-    a = np.ones((256, 2048), np.float32)
-    b = np.ones((2048, 256), np.float32)
-    c = hip.asarray(np.full((256, 256), np.nan, np.float32))
+    a = np.ones((512, 2048), np.float32)
+    b = np.ones((2048, 384), np.float32)
+    c = hip.asarray(np.full((512, 384), np.nan, np.float32))
     ops.gemm(hip.asarray(a), hip.asarray(b), c, 1.0, 0.0)
     assert "_splitk" in mrt.last_kernel()
     assert (c.asnumpy() == 2048).all()
@@ -709,17 +715,19 @@ def test_split_k_beta_zero_ignores_c(env):
     (np.float32, 1536, 1408, 2056, "sgemm_mfma_128x128_even+edges"),  # the rest of K beside
     (np.float32, 1500, 1500, 1200, "sgemm_mfma_128x128_ragged_even"),
     (np.float32, 1000, 1100, 1200, "sgemm_mfma_128x128_ragged_splitk"),  # 72 tiles x 7 on 512 blocks
-    (np.float32, 2000, 2300, 2600, "sgemm_mfma_128x128_ragged_even"),
+    (np.float32, 2000, 2300, 3600, "sgemm_mfma_128x128_ragged_even"),
     # from 192 padded tiles on, ragged float32 shapes run on the large tile over
     # zero-padded copies of both operands: 210 tiles in even shares, 256 as they are
-    (np.float32, 3560, 3800, 1020, "sgemm_mfma_256x256_even+packed"),
-    (np.float32, 4000, 4000, 530, "sgemm_mfma_256x256+packed"),
+    # (K over 3500: under that their parts are split ahead)
+    (np.float32, 3560, 3800, 3600, "sgemm_mfma_256x256_even+packed"),
+    (np.float32, 4000, 4000, 3504, "sgemm_mfma_256x256+packed"),
     (np.float64, 3072, 3072, 512, "dgemm_mfma_128x128_even"),         # 1.125 rounds
     (np.float64, 1536, 1536, 2048, "dgemm_mfma_128x128_even"),        # 144 tiles: 3 slices fill 0.84
     (np.float64, 1500, 1500, 1200, "dgemm_mfma_128x128_ragged_even"),
     # equal slices of K go first where they fill the blocks: 64 tiles x 8, 72 x 7
     (np.float64, 1024, 1024, 4096, "dgemm_mfma_128x128_splitk"),
-    (np.float64, 1000, 1100, 1200, "dgemm_mfma_128x128_ragged_splitk"),  # the reference's preset
+    (np.float64, 1000, 1100, 4000, "dgemm_mfma_128x128_ragged_splitk"),
+    (np.float64, 1000, 1100, 1200, "dgemm_fine"),                     # the reference's preset
     (np.float32, 1152, 1152, 1152, "sgemm_mfma_128x128_splitk"),
     # float64 tiles moved inside the operands; off the word grid from 256 padded
     # tiles on, the same tile over zero-padded copies

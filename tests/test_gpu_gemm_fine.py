@@ -9,8 +9,13 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(scope="module")
 def env(hip):
-    from numba_mlir_amd.mlir import ops
-    return hip, ops
+    from numba_mlir_amd.mlir import math_runtime, ops
+
+    def gemm(*args):
+        ops.gemm(*args)
+        kernel = math_runtime.last_kernel()
+        assert kernel.split("_")[1] == "fine", kernel
+    return hip, gemm
 
 
 def _dev(hip, a, transposed, off):
@@ -39,7 +44,7 @@ SHAPES = [(1, 1, 16), (15, 17, 17), (16, 16, 31), (17, 33, 63), (31, 47, 64), (3
 def test_against_higher_precision(env, dtype, m, n, k):
     """A sum of K products in any order is within K roundings of |a| |b|: K / 2 of
     its last place to nearest."""
-    hip, ops = env
+    hip, gemm = env
     rng = np.random.default_rng(m + 10 * n + 100 * k)
     a, b = rng.standard_normal((m, k)).astype(dtype), rng.standard_normal((k, n)).astype(dtype)
     c0 = rng.standard_normal((m, n)).astype(dtype)
@@ -51,21 +56,21 @@ def test_against_higher_precision(env, dtype, m, n, k):
             for off in (False, True):
                 d_a, d_b = _dev(hip, a, ta, off), _dev(hip, b, tb, off)
                 d_c = hip.asarray(np.full((m, n), np.nan, dtype))
-                ops.gemm(d_a, d_b, d_c, 1.0, 0.0)
+                gemm(d_a, d_b, d_c, 1.0, 0.0)
                 got = d_c.asnumpy()
                 assert (np.abs(got - product) <= bound).all(), (ta, tb, off)
-                ops.gemm(d_a, d_b, d_c, 1.0, 0.0)
+                gemm(d_a, d_b, d_c, 1.0, 0.0)
                 assert np.array_equal(d_c.asnumpy(), got)
     wide = rng.standard_normal((m, n + 2)).astype(dtype)
     d_w = hip.asarray(wide)
-    ops.gemm(d_a, d_b, d_w[:, 1:n + 1], 1.5, -0.5)
+    gemm(d_a, d_b, d_w[:, 1:n + 1], 1.5, -0.5)
     got = d_w.asnumpy()
     assert np.array_equal(got[:, 0], wide[:, 0]) and np.array_equal(got[:, n + 1], wide[:, n + 1])
     want = 1.5 * product - 0.5 * wide[:, 1:n + 1].astype(high)
     room = 1.5 * bound + 4 * np.finfo(dtype).eps * (1.5 * np.abs(product) + np.abs(wide[:, 1:n + 1]))
     assert (np.abs(got[:, 1:n + 1] - want) <= room).all()
     d_t = hip.asarray(np.ascontiguousarray(c0.T)).T      # a column-major C
-    ops.gemm(d_a, d_b, d_t, 1.0, 0.0)
+    gemm(d_a, d_b, d_t, 1.0, 0.0)
     assert (np.abs(d_t.asnumpy() - product) <= bound).all()
 
 
@@ -74,7 +79,7 @@ def test_values_without_a_scaled_form(env, m, n, k):
     """Float32 operands among the largest and the smallest numbers, infinities and
     NaN: what plain float32 arithmetic gives, and a sum among the subnormal numbers
     within one rounding of each wave's part of it."""
-    hip, ops = env
+    hip, gemm = env
     rng = np.random.default_rng(k)
     a0 = rng.standard_normal((m, k), dtype=np.float32)
     b0 = rng.standard_normal((k, n), dtype=np.float32)
@@ -83,7 +88,7 @@ def test_values_without_a_scaled_form(env, m, n, k):
 
     def run(a, b):
         d_c = hip.asarray(np.full((m, n), np.nan, np.float32))
-        ops.gemm(hip.asarray(a), hip.asarray(b), d_c, 1.0, 0.0)
+        gemm(hip.asarray(a), hip.asarray(b), d_c, 1.0, 0.0)
         return d_c.asnumpy()
 
     for ea, eb in ((110, 0), (0, 100), (60, 50), (-70, -66), (-140, 20), (20, -145)):

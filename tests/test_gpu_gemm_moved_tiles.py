@@ -12,10 +12,11 @@ pytestmark = pytest.mark.gpu
                                       (False, True, False), (True, True, False),
                                       (False, False, True), (True, True, True)])
 @pytest.mark.parametrize("m,n,k", [
-    (128, 2050, 18), (2049, 128, 34), (130, 132, 2050),     # one tile across, slices of K
-    (514, 516, 15), (515, 1031, 17), (640, 513, 33),        # odd extents go through copies
-    (1028, 1030, 1026), (1500, 1502, 606),                  # slices, shares
-    (2050, 2052, 270), (2048, 2048, 270),                   # 289 tiles; only K is cut short
+    # (K under 16 or 4e9 products and more: between them small tiles share out K)
+    (128, 2050, 14), (2049, 128, 15), (386, 516, 20402),    # one tile across; slices of K
+    (514, 516, 15), (515, 1031, 13), (640, 513, 9),         # odd extents go through copies
+    (1028, 1030, 3802), (1500, 1502, 1802),                 # slices, shares
+    (2050, 2052, 970), (2048, 2048, 970),                   # 289 tiles; only K is cut short
 ])
 def test_products_of_whole_numbers(hip, m, n, k, ta, tb, tc):
     from numba_mlir_amd.mlir import math_runtime, ops
@@ -35,10 +36,10 @@ def test_products_of_whole_numbers(hip, m, n, k, ta, tb, tc):
 
 @pytest.mark.parametrize("dtype,m,n,k,kernel", [
     # rounds of whole tiles first, then one to two rounds in shares
-    (np.float64, 4100, 4100, 130, "dgemm_mfma_128x128_ragged_even"),      # 1089 tiles: 2.1 rounds
-    (np.float64, 4096, 4224, 144, "dgemm_mfma_128x128_even"),             # 1056 whole tiles
+    (np.float64, 4100, 4100, 242, "dgemm_mfma_128x128_ragged_even"),      # 1089 tiles: 2.1 rounds
+    (np.float64, 4096, 4224, 240, "dgemm_mfma_128x128_even"),             # 1056 whole tiles
     (np.float32, 6144, 6144, 160, "sgemm_mfma_256x256_even"),             # 576: 2.25
-    (np.float32, 6100, 6000, 272, "sgemm_mfma_256x256_even+packed"),
+    (np.float32, 6100, 6000, 3520, "sgemm_mfma_256x256_even+packed"),
     (np.float32, 5888, 8192, 144, "sgemm_mfma_256x256"),                  # 736: 0.96 full, whole
 ])
 @pytest.mark.parametrize("tc", [False, True])

@@ -23,16 +23,18 @@ def _dev(hip, a, transposed, off):
 # (rows and columns one more or less than whole tiles of 128; K of one more or less
 # than slabs of 16 and runs of 4, 8 and 16; a round not full, whole rounds with a
 # few tiles in shares of one slab and more, shares alone, several rounds)
-SHAPES = [(1801, 1300, 433), (3071, 1025, 385), (2047, 2049, 1025), (3329, 3199, 129),
-          (3201, 3327, 191), (1793, 1283, 3499), (129, 20001, 700), (2052, 2180, 516),
-          (1153, 3584, 769), (4481, 4353, 257), (2176, 2045, 256)]
+# (and which of them go in shares)
+SHAPES = [(1801, 1300, 433, ""), (3071, 1025, 385, ""), (2047, 2049, 1025, "_even"),
+          (3329, 3199, 129, ""), (3201, 3327, 191, ""), (1793, 1283, 3499, "_even"),
+          (129, 20001, 700, "_even"), (2052, 2180, 516, "_even"), (1153, 3584, 769, "_even"),
+          (4481, 4353, 257, ""), (2176, 2045, 256, "")]
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
-def test_whole_numbers(hip, m, n, k):
+@pytest.mark.parametrize("m,n,k,shares", SHAPES)
+def test_whole_numbers(hip, m, n, k, shares):
     """Sums below 2^24: exact in any order.  alpha and beta once, nothing written
     beside C, the same bits again."""
-    from numba_mlir_amd.mlir import ops
+    from numba_mlir_amd.mlir import math_runtime, ops
     rng = np.random.default_rng(m + n + k)
     a = rng.integers(-9, 9, (m, k), endpoint=True).astype(np.float32)
     b = rng.integers(-9, 9, (k, n), endpoint=True).astype(np.float32)
@@ -42,6 +44,7 @@ def test_whole_numbers(hip, m, n, k):
         d_a, d_b = _dev(hip, a, ta, off), _dev(hip, b, tb, off)
         d_c = hip.asarray(np.full((m, n), np.nan, np.float32))
         ops.gemm(d_a, d_b, d_c, 1.0, 0.0)
+        assert math_runtime.last_kernel() == "sgemm_planes" + shares
         assert np.array_equal(d_c.asnumpy(), product), (ta, tb, off)
     wide = rng.integers(-99, 99, (m, n + 2), endpoint=True).astype(np.float32)
     d_w = hip.asarray(wide)

@@ -94,7 +94,7 @@ def test_operands_off_the_word_grid_stay_on_tiles_and_edges(gemm_entry_points):
     a 128-bit word into its workspace; this one cannot, and runs the whole
     tiles on the matrix cores and the rest on the strided kernel."""
     hip, lib, mrt = gemm_entry_points
-    m, n, k = 1540, 2052, 1001
+    m, n, k = 1536, 1412, 1001
     rng = np.random.default_rng(5)
     a_wide = rng.standard_normal((m, k + 3), dtype=np.float32)
     b = rng.standard_normal((k, n), dtype=np.float32)
