@@ -108,34 +108,42 @@ template <typename T, int R, bool K_CONTIG> struct FineFetch {
 // only what no other tile has; the end of K is the last 16 of it, without what
 // the whole chunks had.
 //
-// part: slices of sliceK of K along grid.y leave their sums, unscaled, in
-// part[slice][M][ldw] for gemm_splitk_fold.
+// part: slices of sliceK of K leave their sums, unscaled, in part[slice][M][ldw] for
+// gemm_splitk_fold, or gemm_thin_fold if there are more than kFineFewSlices.
 //
-// Blocks that run side by side on one XCD take neighbouring tiles: an XCD's L2
-// then holds an eighth of A's rows.
+// The tiles of all slices, slice by slice, go to the XCDs in eight equal stretches
+// (grid: tiles * slices to a multiple of 8): neighbours, which run side by side, share
+// operands in an XCD's L2, and no XCD has more than an eighth.  (An eighth of the tiles with all
+// their slices each: one tile keeps to one XCD, 32 x 32 x 10^6 float32 218 us instead of
+// 68; six of 42 tiles in six slices are 36 blocks for 32 CUs, 193 x 265 x 47979
+// float64 288 instead of 148.)
+constexpr int kFineFewSlices = 8;
 template <typename T, int RM, int RN, int W, int WAVES, bool A_KC, bool B_NC>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(WAVES))) void
 gemm_fine(const T *__restrict__ A, const T *__restrict__ B, T *__restrict__ C, int M, int N,
           int K, int64_t lda, int64_t ldb, int64_t ldc, T alpha, T beta, int tiles, int tilesN,
-          int sliceK, T *__restrict__ part, int64_t ldw) {
+          int slices, int sliceK, T *__restrict__ part, int64_t ldw) {
   typedef typename FineMma<T>::Acc Acc;
   typedef FineFetch<T, RM, A_KC> FetchA;
   typedef FineFetch<T, RN, !B_NC> FetchB;
   constexpr int CK = 16, RUN = sizeof(T) == 4 ? 4 : 10, BM = 16 * RM, BN = 16 * RN, REGS = RM * RN * 4;
   __shared__ T sums[W][REGS][64];
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-  const int perXcd = (tiles + 7) / 8;
-  const int tile = int(blockIdx.x % 8) * perXcd + int(blockIdx.x / 8);
-  if (tile >= tiles)
+  int tile = int(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8), slice = 0;
+  if (part) {
+    slice = int(uint32_t(tile) / uint32_t(tiles));
+    tile -= slice * tiles;
+  }
+  if (slice >= slices || tile >= tiles)
     return;
   const int bm = tile / tilesN * BM, bn = tile % tilesN * BN;
   const int m0 = RM > 1 && bm > M - BM ? M - BM : bm, n0 = RN > 1 && bn > N - BN ? N - BN : bn;
   if (part) {
-    const int k0 = blockIdx.y * sliceK;
+    const int k0 = slice * sliceK;
     A += A_KC ? int64_t(k0) : int64_t(k0) * lda;
     B += B_NC ? int64_t(k0) * ldb : int64_t(k0);
     K = K - k0 < sliceK ? K - k0 : sliceK;
-    C = part + int64_t(blockIdx.y) * M * ldw;
+    C = part + int64_t(slice) * M * ldw;
     ldc = ldw;
     alpha = T(1);
     beta = T(0);

@@ -583,9 +583,10 @@ def test_small_products_of_long_operands(env, dtype, k, m, n):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("m,k,n", [(16, 1 << 18, 16), (32, 100_003, 20), (100, 200_000, 60),
-                                   (128, 1 << 17, 128), (300, 1 << 15, 300), (10, 4099, 12)])
-def test_few_tiles_with_a_long_k(env, dtype, m, k, n):
+@pytest.mark.parametrize("m,k,n,kernel", [(16, 1 << 18, 16, "fine"), (32, 100_003, 20, "fine"),
+                                          (100, 50_000, 60, "gemm"), (128, 1 << 18, 128, "mfma"),
+                                          (300, 1 << 16, 300, "mfma"), (10, 4099, 12, "fine")])
+def test_few_tiles_with_a_long_k(env, dtype, m, k, n, kernel):
     """Results of a few tiles from long operands: K is cut into slices, on
     the tiles of 16 to 48 rows for the smallest results and on the guarded tiles
     from a quarter of a tile on."""
@@ -599,7 +600,7 @@ def test_few_tiles_with_a_long_k(env, dtype, m, k, n):
         d_c = hip.asarray(c0)
         ops.gemm(d_a, hip.asarray(b), d_c, 1.5, -0.5)
         assert "_splitk" in mrt.last_kernel(), mrt.last_kernel()
-        assert ("fine" in mrt.last_kernel()) == (m * n < 4096)
+        assert kernel in mrt.last_kernel()
         _check_scaled(d_c.asnumpy(), a, b, c0, 1.5, -0.5, tol)
 
 

@@ -15,6 +15,7 @@ def env(hip):
         ops.gemm(*args)
         kernel = math_runtime.last_kernel()
         assert kernel.split("_")[1] == "fine", kernel
+        return kernel
     return hip, gemm
 
 
@@ -32,7 +33,7 @@ def _dev(hip, a, transposed, off):
 
 # (no tile, one tile, one row or column more or less than whole tiles of 16, 32 and
 # 48; K of one chunk of 16 and one more or less than whole chunks of 4 and 8 waves,
-# of a run and of slices; the last ones the longest that slices of K take)
+# of a run and of slices)
 SHAPES = [(1, 1, 16), (15, 17, 17), (16, 16, 31), (17, 33, 63), (31, 47, 64), (33, 49, 65),
           (47, 33, 129), (49, 97, 255), (97, 49, 257), (310, 1, 506), (1, 127, 1000),
           (200, 300, 641), (129, 143, 1025), (500, 350, 33), (1000, 1100, 80), (64, 48, 5000),
@@ -72,6 +73,57 @@ def test_against_higher_precision(env, dtype, m, n, k):
     d_t = hip.asarray(np.ascontiguousarray(c0.T)).T      # a column-major C
     gemm(d_a, d_b, d_t, 1.0, 0.0)
     assert (np.abs(d_t.asnumpy() - product) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m,n,k", [(9, 9, 100_003), (16, 16, 2064), (31, 33, 50_021), (63, 63, 9000),
+                                   (20, 150, 4113), (1, 63, 70_001), (48, 85, 16_411)])
+def test_many_slices_of_a_long_k(env, dtype, m, n, k):
+    """Small results of a long K in 16 slices and more, the last one shorter or
+    longer by a few: every element within its products' roundings, alpha and beta
+    once, nothing beside C, the same bits again."""
+    hip, gemm = env
+    rng = np.random.default_rng(m + n + k)
+    a, b = rng.standard_normal((m, k)).astype(dtype), rng.standard_normal((k, n)).astype(dtype)
+    high = np.float64 if dtype == np.float32 else np.longdouble
+    product = a.astype(high) @ b.astype(high)
+    bound = (k + 4) * np.finfo(dtype).eps / 2 * (np.abs(a).astype(high) @ np.abs(b).astype(high))
+    wide = rng.standard_normal((m, n + 2)).astype(dtype)
+    for ta in (False, True):
+        for tb in (False, True):
+            d_a, d_b = _dev(hip, a, ta, ta == tb), _dev(hip, b, tb, ta == tb)
+            outs = []
+            for _ in range(2):
+                d_c = hip.asarray(np.full((m, n), np.nan, dtype))
+                assert gemm(d_a, d_b, d_c, 1.0, 0.0).endswith("_fine_splitk")
+                outs.append(d_c.asnumpy())
+            assert np.array_equal(outs[0], outs[1])
+            assert (np.abs(outs[0] - product) <= bound).all(), (ta, tb)
+    d_w = hip.asarray(wide)
+    gemm(d_a, d_b, d_w[:, 1:n + 1], 1.5, -0.5)
+    got = d_w.asnumpy()
+    assert np.array_equal(got[:, 0], wide[:, 0]) and np.array_equal(got[:, n + 1], wide[:, n + 1])
+    want = 1.5 * product - 0.5 * wide[:, 1:n + 1].astype(high)
+    room = 1.5 * bound + 4 * np.finfo(dtype).eps * (1.5 * np.abs(product) + np.abs(wide[:, 1:n + 1]))
+    assert (np.abs(got[:, 1:n + 1] - want) <= room).all()
+
+
+def test_a_long_k_fills_the_gpu(env):
+    """32 x 32 from a million of K: 55 to 68 us in slices on all XCDs, 140 on the
+    strided kernel in slices, 350 and more in eight slices on one XCD."""
+    import time
+    hip, gemm = env
+    m = n = 32
+    k = 1_000_000
+    d_a = hip.asarray(np.ones((k, m), np.float32)).T
+    d_b, d_c = hip.asarray(np.ones((k, n), np.float32)), hip.asarray(np.zeros((m, n), np.float32))
+    times = []
+    for _ in range(20):
+        start = time.perf_counter()
+        gemm(d_a, d_b, d_c, 1.0, 0.0)
+        times.append(time.perf_counter() - start)
+    assert (d_c.asnumpy() == k).all()
+    assert min(times) < 200e-6
 
 
 @pytest.mark.parametrize("m,n,k", [(40, 50, 70), (100, 130, 300), (300, 200, 150)])
