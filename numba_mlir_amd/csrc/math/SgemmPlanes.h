@@ -207,18 +207,16 @@ sgemm_planes(const uintx4 *__restrict__ A, const uintx4 *__restrict__ B, float *
   const uintx4 *a0 = A, *b0 = B;
   // The n-th KiB of a wave's part of a slab of both operands on its way to LDS.
   // (Inline assembly, so that the waits are those written here: the compiler
-  // lets every LDS read wait for all such loads.  They write LDS alone; m0, which
-  // cannot be declared as written, is put back.)
+  // lets every LDS read wait for all such loads.  They write LDS alone, from the
+  // address in m0 on, which the compiler puts there.)
   auto fetch = [&](int n, int s, int stage) {
     const bool left = n < NA;
     const uint32_t to = ldsAddress(left ? As[stage] : Bs[stage]) +
                         16 * (wave * 64 + THREADS * (left ? n : n - NA));
     const uintx4 *from = (left ? a0 : b0) + int64_t(s) * kPlanesWords;
-    uint32_t m0;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
-                 "global_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
-                 : "=&s"(m0)
-                 : "s"(to), "v"(left ? fromA[left ? n : 0] : fromB[left ? 0 : n - NA]), "s"(from)
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "{m0}"(to), "v"(left ? fromA[left ? n : 0] : fromB[left ? 0 : n - NA]), "s"(from)
                  : "memory");
   };
   // A segment's first slabs on their way; no wave reads LDS any more.
