@@ -37,11 +37,17 @@ constexpr int kPlaneWords = 64, kPlanesWords = 3 * kPlaneWords;
 // Element (r, k) of the operand is src[r * rowStride + k * kStride]; one of the
 // strides is one.  rowTiles x slabs tiles are written, zero beyond R and K; run:
 // slabs of every second run of so many have their sign changed (0: none).
+//
+// A tile of 32 rows and a slab that holds an infinity, a NaN or an element too large
+// for parts is left out (its parts are zero) and flagged, a byte each in
+// flags[rowTile / 4][slab][rowTile % 4]: the product kernel adds what it is part of
+// from the operands themselves.
 struct PlanesJob {
   const float *src;
   int64_t rowStride, kStride;
   int R, K, rowTiles, slabs, run;
   uintx4 *dst;
+  unsigned char *flags;
   __host__ __device__ int64_t blocks() const { return int64_t(rowTiles) * ((slabs + 3) / 4); }
 };
 
@@ -81,15 +87,26 @@ __global__ __launch_bounds__(256) void sgemm_split_planes(PlanesJob first, Plane
     for (int j = 0; j < 8; ++j)
       v[j] = r < job.R && k + j < job.K ? at[j * job.kStride] : 0.0f;
   }
+  uint32_t largest = 0; // of the values' bits without their sign
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    v[j] *= scale;
+    const uint32_t bits = __builtin_bit_cast(uint32_t, v[j]) & 0x7fffffffu;
+    largest = bits > largest ? bits : largest;
+  }
+  // (what rounds to infinity as a bf16, and all beyond)
+  const bool flag = __builtin_amdgcn_ballot_w64(largest >= 0x7f7f8000u) != 0;
   uintx4 h, m, l;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     uint32_t ph, pm, pl;
-    partsOf(scale * v[2 * j], scale * v[2 * j + 1], ph, pm, pl);
+    partsOf(flag ? 0.0f : v[2 * j], flag ? 0.0f : v[2 * j + 1], ph, pm, pl);
     h[j] = ph;
     m[j] = pm;
     l[j] = pl;
   }
+  if (lane == 0)
+    job.flags[(int64_t(tile / 4) * job.slabs + slab) * 4 + tile % 4] = flag;
   uintx4 *to = job.dst + (int64_t(tile) * job.slabs + slab) * kPlanesWords + lane;
   to[0] = h;
   to[kPlaneWords] = m;
@@ -107,12 +124,15 @@ __host__ __device__ inline void panelTile(int64_t tile, int tilesM, int tilesN, 
   tn = int(p * uint32_t(panel) + in % width);
 }
 
-// The operands as they are, for the tiles that the parts cannot compute.
+// The operands as they are, for what the parts cannot compute, and what that is: a
+// word for each 128 rows and slab, a byte of it for each 32 rows.
 struct PlanesSource {
   const float *X, *Y;
   int64_t xm, xk, yk, yn;
   int K;
+  const uint32_t *xFlags, *yFlags;
 };
+constexpr int kPlanesMostSlabs = 256; // of a tile: a thread looks at the flags of one
 
 __device__ __forceinline__ uint32_t ldsAddress(const uintx4 *p) {
   return uint32_t(
@@ -205,6 +225,7 @@ sgemm_planes(const uintx4 *__restrict__ A, const uintx4 *__restrict__ B, float *
   PlanesSegment seg = walk.next(plan, G);
   int bm = 0, bn = 0, slab0 = 0, slab1 = 0;
   const uintx4 *a0 = A, *b0 = B;
+  uint32_t flagA = 0, flagB = 0; // of slab tid of the segment
   // The n-th KiB of a wave's part of a slab of both operands on its way to LDS.
   // (Inline assembly, so that the waits are those written here: the compiler
   // lets every LDS read wait for all such loads.  They write LDS alone, from the
@@ -229,6 +250,11 @@ sgemm_planes(const uintx4 *__restrict__ A, const uintx4 *__restrict__ B, float *
     slab1 = seg.slab1;
     a0 = A + int64_t(bm / 32) * slabs * kPlanesWords;
     b0 = B + int64_t(bn / 32) * slabs * kPlanesWords;
+    flagA = flagB = 0; // (loaded ahead of the slabs: behind them a tile would wait for it)
+    if (tid >= slab0 && tid < slab1) {
+      flagA = src.xFlags[int64_t(tm) * slabs + tid];
+      flagB = src.yFlags[int64_t(tn) * slabs + tid];
+    }
 #pragma unroll
     for (int i = 0; i < STAGES; ++i)
       if (slab0 + i < slab1) {
@@ -271,6 +297,11 @@ sgemm_planes(const uintx4 *__restrict__ A, const uintx4 *__restrict__ B, float *
           }
     };
     int cur = 0; // the stage of the slab that is multiplied
+    const bool inside = tid >= slab0 && tid < slab1;
+    auto flagsHere = [&] { // (waited for here, not before the tile)
+      asm volatile("" : "+v"(flagA), "+v"(flagB));
+      return (flagA | flagB) != 0;
+    };
 
     struct Operands {
       bf16x8 a[TM][3], b[TN][3];
@@ -371,7 +402,13 @@ sgemm_planes(const uintx4 *__restrict__ A, const uintx4 *__restrict__ B, float *
       }
       flush(s - 1);
       if (s >= look && s < slab1) {
-        early = __syncthreads_or(2 * __builtin_popcount(tilesLost()) > TM * TN);
+        // (or most of the slabs are flagged)
+        const bool many = 2 * __builtin_popcount(tilesLost()) > TM * TN;
+        const uint64_t flagged = __builtin_amdgcn_ballot_w64(flagsHere());
+        const uint64_t all = __builtin_amdgcn_ballot_w64(inside);
+        if (__syncthreads_or(many || flagged))
+          early = __syncthreads_or(many) ||
+                  __syncthreads_and(2 * __builtin_popcountll(flagged) >= __builtin_popcountll(all));
         look = s + 128;
       }
     }
@@ -387,89 +424,113 @@ sgemm_planes(const uintx4 *__restrict__ A, const uintx4 *__restrict__ B, float *
                              ? 0.0f
                              : __builtin_fmaf(sum[i][j][r], 1.0f / (kPartsScale * kPartsScale),
                                               0.0f); // (no -0)
-    if (__syncthreads_or(lost != 0)) {
-      // The lost tiles with v_mfma_f32_32x32x2_f32 on the operands themselves:
-      // lane half h of the wave takes k = 8 h + t of the slab in step t.  In LDS a
-      // row's 16 of a slab are [half of K][row][two words]; the next slab is loaded
-      // while one is multiplied.  2047 x 2049 x 2051, us a call, on sgemm_parts / loads in
-      // their slab / this: all sums too large 281 / 466 / 295, an infinity in the last
-      // column of every 128th row 240 / 469 / 300 and of every row 303 / 531 / 361 (one
-      // wave a SIMD has no other to run beside its waits).
-      constexpr int NX = 4 * BM / THREADS, NY = 4 * BN / THREADS;
-      static_assert(4 * BM % THREADS == 0 && 4 * BN % THREADS == 0, "whole quads a thread");
-      floatx4 x[NX], y[NY];
-      const float *atX[NX], *atY[NY]; // of k = 4 quad; the last row stands for those beyond
-      auto place = [&](int n, int rows, int64_t kStride, int &row, int &quad) {
-        const int w = tid + THREADS * n;
-        quad = kStride == 1 ? w % 4 : w / rows;
-        row = kStride == 1 ? w / 4 : w % rows;
-      };
-      auto start = [&](auto &at, int rows, const float *p, int64_t rowStride, int64_t kStride,
-                       int origin, int extent) {
-#pragma unroll
-        for (int n = 0; n < int(sizeof(at) / sizeof(at[0])); ++n) {
-          int row, quad;
-          place(n, rows, kStride, row, quad);
-          const int r = origin + row < extent ? origin + row : extent - 1;
-          at[n] = p + r * rowStride + 4 * quad * kStride;
-        }
-      };
-      auto load = [&](auto &v, const auto &at, int rows, int64_t kStride, int k0) {
-#pragma unroll
-        for (int n = 0; n < int(sizeof(at) / sizeof(at[0])); ++n) {
-          if (k0 + 16 <= src.K) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              v[n][q] = at[n][(k0 + q) * kStride];
-          } else {
-            int row, quad;
-            place(n, rows, kStride, row, quad);
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              v[n][q] = k0 + 4 * quad + q < src.K ? at[n][(k0 + q) * kStride] : 0.0f;
+    const bool flag = flagsHere();
+    if (__syncthreads_or(lost != 0 || flag)) {
+      // The lost tiles, and the flagged slabs of the others, with
+      // v_mfma_f32_32x32x2_f32 on the operands themselves: lane half h of the wave takes
+      // k = 8 h + t of the slab in step t.  In LDS a slab is [four of K][row], rows so
+      // that neither four apart nor side by side share a bank.  Waves 0 and 1 load A's
+      // rows, 2 and 3 B's, a thread four rows by four of K in four words, four slabs
+      // ahead in registers (one wave a SIMD has no other to run beside its waits).
+      //
+      // us a call, on sgemm_parts / whole tiles again, a slab ahead / this: 2047 x 2049 x
+      // 2051 (ordinary data 147 / 133 / 134) one NaN 178 / 297 / 136, an infinity in the
+      // last column of every 128th row 220 / 319 / 141 and of every row 288 / 398 / 141,
+      // all sums too large 248 / 315 / 244; 1801 x 1300 x 433 (46 / 43 / 43) 48 / 77 / 46,
+      // 50 / 74 / 45, 53 / 86 / 46, 68 / 86 / 77.
+      static_assert(BM == 128 && BN == 128 && STAGES == 4, "four by four a thread, four ahead");
+      constexpr int QUAD = 148; // words of four of K
+      auto placeOf = [](int row) { return row % 4 * 34 + row / 4; };
+      uint32_t *flags = reinterpret_cast<uint32_t *>(As[0] + 4 * QUAD); // A's, then B's
+      uint64_t *need = reinterpret_cast<uint64_t *>(flags + 2 * kPlanesMostSlabs);
+      static_assert((AW - 4 * QUAD) * 16 >= 8 * kPlanesMostSlabs + 8 * THREADS / 64 &&
+                        THREADS == kPlanesMostSlabs,
+                    "room behind the slab; a flag a thread");
+      const bool whole = __syncthreads_or(lost != 0); // all slabs, not the flagged ones alone
+      const uint64_t bits = __builtin_amdgcn_ballot_w64(inside && (whole || flag));
+      flags[tid] = flagA;
+      flags[kPlanesMostSlabs + tid] = flagB;
+      if (lane == 0)
+        need[wave] = bits;
+      __syncthreads();
+      auto uniform = [](uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); };
+      const int full = src.K / 16, end = slab1 < full ? slab1 : full; // whole slabs
+      auto following = [&](int k) { // the next slab after k, or end
+        for (++k; k < end; k = (k | 63) + 1) {
+          const uint64_t word = need[k >> 6] >> (k & 63);
+          const uint64_t rest = uint64_t(uniform(uint32_t(word >> 32))) << 32 |
+                                uniform(uint32_t(word));
+          if (rest) {
+            k += __builtin_ctzll(rest);
+            break;
           }
         }
+        return k < end ? k : end;
       };
-      auto stash = [&](const auto &v, uintx4 *lds, int rows, int64_t kStride) {
+      const bool forA = wave < 2;
+      const int64_t rowStride = forA ? src.xm : src.yn, kStride = forA ? src.xk : src.yk;
+      const int origin = forA ? bm : bn, extent = forA ? M : N;
+      const bool kContig = kStride == 1, ragged = !kContig && origin + BM > extent;
+      // (its rows: kContig row, row + 32, ..., else row, row + 1, ...)
+      const int quad = kContig ? tid % 4 : tid % 128 / 32;
+      const int row = kContig ? tid % 128 / 4 : 4 * (tid % 32);
+      const int r0 = origin + row, r4 = r0 < extent - 4 ? r0 : extent - 4;
+      const int shift = r0 - r4 < 3 ? r0 - r4 : 3; // (rows beyond the last are the last again)
+      const float *at[4];
 #pragma unroll
-        for (int n = 0; n < int(sizeof(v) / sizeof(v[0])); ++n) {
-          int row, quad;
-          place(n, rows, kStride, row, quad);
-          reinterpret_cast<floatx4 *>(lds)[2 * (quad / 2 * rows + row) + quad % 2] = v[n];
+      for (int i = 0; i < 4; ++i) {
+        const int r = r0 + 32 * i < extent ? r0 + 32 * i : extent - 1;
+        at[i] = (forA ? src.X : src.Y) + (kContig ? int64_t(r) * rowStride + 4 * quad
+                                                  : r4 + int64_t(4 * quad + i) * kStride);
+      }
+      typedef FineElems<float, 4> Word;
+      auto load = [&](floatx4 (&v)[4], int k) {
+        k = k < end ? k : full - 1; // (nothing more: loaded in vain, so that no load is in a branch)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const Word w = *reinterpret_cast<const Word *>(at[i] + int64_t(k) * (16 * kStride));
+          v[i] = floatx4{w.v[0], w.v[1], w.v[2], w.v[3]};
         }
       };
-      start(atX, BM, src.X, src.xm, src.xk, bm, M);
-      start(atY, BN, src.Y, src.yn, src.yk, bn, N);
-      auto loadBoth = [&](int s) {
-        load(x, atX, BM, src.xk, 16 * s);
-        load(y, atY, BN, src.yk, 16 * s);
+      auto stash = [&](floatx4 (&v)[4], int stage) {
+        if (ragged) {
+#pragma unroll
+          for (int by = 1; by <= 2; ++by)
+            if (shift & by) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  v[i][e] = v[i][e + by < 3 ? e + by : 3];
+            }
+        }
+        floatx4 *to = reinterpret_cast<floatx4 *>(forA ? As[stage] : Bs[stage]) +
+                      quad * QUAD + placeOf(row);
+        const int apart = kContig ? placeOf(32) : placeOf(1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          to[i * apart] = kContig ? v[i] : floatx4{v[0][i], v[1][i], v[2][i], v[3][i]};
       };
-      loadBoth(slab0);
-#pragma nounroll
-      for (s = slab0; s < slab1; ++s) {
-        const int cur = (s - slab0) & 1;
-        stash(x, As[cur], BM, src.xk);
-        stash(y, Bs[cur], BN, src.yk);
-        __syncthreads(); // (also: every wave has read the slab before the last)
-        if (s + 1 < slab1)
-          loadBoth(s + 1);
+      auto add = [&](int k, int stage) {
         floatx4 left[TM][2], right[TN][2];
 #pragma unroll
         for (int w = 0; w < 2; ++w) {
 #pragma unroll
           for (int i = 0; i < TM; ++i)
             left[i][w] = reinterpret_cast<const floatx4 *>(
-                As[cur])[2 * (lane / 32 * BM + (wm * TM + i) * 32 + lane % 32) + w];
+                As[stage])[(lane / 32 * 2 + w) * QUAD + placeOf((wm * TM + i) * 32 + lane % 32)];
 #pragma unroll
           for (int j = 0; j < TN; ++j)
             right[j][w] = reinterpret_cast<const floatx4 *>(
-                Bs[cur])[2 * (lane / 32 * BN + (wn * TN + j) * 32 + lane % 32) + w];
+                Bs[stage])[(lane / 32 * 2 + w) * QUAD + placeOf((wn * TN + j) * 32 + lane % 32)];
         }
+        const uint32_t fa = uniform(flags[k]) >> (8 * TM * wm);
+        const uint32_t fb = uniform(flags[kPlanesMostSlabs + k]) >> (8 * TN * wn);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
           for (int j = 0; j < TN; ++j) {
-            if (!(lost >> (i * TN + j) & 1))
+            if (!(lost >> (i * TN + j) & 1 || (fa >> (8 * i) & 1) || (fb >> (8 * j) & 1)))
               continue;
 #pragma unroll
             for (int t = 0; t < 8; ++t)
@@ -477,6 +538,46 @@ sgemm_planes(const uintx4 *__restrict__ A, const uintx4 *__restrict__ B, float *
                                                                right[j][t / 4][t % 4], sum[i][j],
                                                                0, 0, 0);
           }
+      };
+      // (waits for LDS alone: loads stay on their way)
+      auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); };
+      floatx4 v0[4], v1[4], v2[4], v3[4];
+      int next = following(slab0 - 1), k0, k1, k2, k3; // the slab after those in v0 to v3
+      auto start = [&](floatx4 (&v)[4], int &k) {
+        load(v, k = next);
+        next = following(next);
+      };
+      auto step = [&](floatx4 (&v)[4], int &k, int stage) {
+        stash(v, stage);
+        meet(); // (also: every wave has read the stage of three slabs before)
+        const int of = k;
+        start(v, k);
+        if (of < end)
+          add(of, stage);
+      };
+      start(v0, k0);
+      start(v1, k1);
+      start(v2, k2);
+      start(v3, k3);
+#pragma nounroll
+      while (k0 < end) { // (four steps without a way out between: see load)
+        step(v0, k0, 0);
+        step(v1, k1, 1);
+        step(v2, k2, 2);
+        step(v3, k3, 3);
+      }
+      if (slab1 > full && need[full >> 6] >> (full & 63) & 1) { // the end of K
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            v0[i][e] = 16 * full + 4 * quad + (kContig ? e : i) < src.K
+                               ? at[i][int64_t(full) * (16 * kStride) + e]
+                               : 0.0f;
+        __syncthreads();
+        stash(v0, 0);
+        __syncthreads();
+        add(full, 0);
       }
     }
 
