@@ -439,6 +439,9 @@ sgemm_planes(const uintx4 *__restrict__ A, const uintx4 *__restrict__ B, float *
       // all sums too large 248 / 315 / 244; 1801 x 1300 x 433 (46 / 43 / 43) 48 / 77 / 46,
       // 50 / 74 / 45, 53 / 86 / 46, 68 / 86 / 77.
       static_assert(BM == 128 && BN == 128 && STAGES == 4, "four by four a thread, four ahead");
+      int here = tid; // (places are worked out here, not ahead of the tiles)
+      asm volatile("" : "+v"(here));
+      const int home = here % 64;
       constexpr int QUAD = 148; // words of four of K
       auto placeOf = [](int row) { return row % 4 * 34 + row / 4; };
       uint32_t *flags = reinterpret_cast<uint32_t *>(As[0] + 4 * QUAD); // A's, then B's
@@ -448,8 +451,8 @@ sgemm_planes(const uintx4 *__restrict__ A, const uintx4 *__restrict__ B, float *
                     "room behind the slab; a flag a thread");
       const bool whole = __syncthreads_or(lost != 0); // all slabs, not the flagged ones alone
       const uint64_t bits = __builtin_amdgcn_ballot_w64(inside && (whole || flag));
-      flags[tid] = flagA;
-      flags[kPlanesMostSlabs + tid] = flagB;
+      flags[here] = flagA;
+      flags[kPlanesMostSlabs + here] = flagB;
       if (lane == 0)
         need[wave] = bits;
       __syncthreads();
@@ -472,8 +475,8 @@ sgemm_planes(const uintx4 *__restrict__ A, const uintx4 *__restrict__ B, float *
       const int origin = forA ? bm : bn, extent = forA ? M : N;
       const bool kContig = kStride == 1, ragged = !kContig && origin + BM > extent;
       // (its rows: kContig row, row + 32, ..., else row, row + 1, ...)
-      const int quad = kContig ? tid % 4 : tid % 128 / 32;
-      const int row = kContig ? tid % 128 / 4 : 4 * (tid % 32);
+      const int quad = kContig ? here % 4 : here % 128 / 32;
+      const int row = kContig ? here % 128 / 4 : 4 * (here % 32);
       const int r0 = origin + row, r4 = r0 < extent - 4 ? r0 : extent - 4;
       const int shift = r0 - r4 < 3 ? r0 - r4 : 3; // (rows beyond the last are the last again)
       const float *at[4];
@@ -518,11 +521,11 @@ sgemm_planes(const uintx4 *__restrict__ A, const uintx4 *__restrict__ B, float *
 #pragma unroll
           for (int i = 0; i < TM; ++i)
             left[i][w] = reinterpret_cast<const floatx4 *>(
-                As[stage])[(lane / 32 * 2 + w) * QUAD + placeOf((wm * TM + i) * 32 + lane % 32)];
+                As[stage])[(home / 32 * 2 + w) * QUAD + placeOf((wm * TM + i) * 32 + home % 32)];
 #pragma unroll
           for (int j = 0; j < TN; ++j)
             right[j][w] = reinterpret_cast<const floatx4 *>(
-                Bs[stage])[(lane / 32 * 2 + w) * QUAD + placeOf((wn * TN + j) * 32 + lane % 32)];
+                Bs[stage])[(home / 32 * 2 + w) * QUAD + placeOf((wn * TN + j) * 32 + home % 32)];
         }
         const uint32_t fa = uniform(flags[k]) >> (8 * TM * wm);
         const uint32_t fb = uniform(flags[kPlanesMostSlabs + k]) >> (8 * TN * wn);
