@@ -31,6 +31,16 @@ def _dev(hip, a, transposed, off):
     return view.T if transposed else view
 
 
+def _norm_room(dtype, k):
+    """2-norm of the error over that of a product of normal operands: the i-th of n
+    roundings in turn moves a sum of size sqrt(i) by 2^-p / sqrt(3) of it in the mean, all of
+    them together by 2^-p sqrt(n / 6) of the whole; no sum in registers has more than 64
+    terms (float32) or 160, and those sums' own sum, the slices' and the scale have another
+    2^-p.  (Measured 1.0 to 3.6 2^-24 and 1.3 to 4.5 2^-53, of 2.6 to 4.3 and to 6.2.  Operands
+    of 16 bits are far beyond; sums left in the registers 5.2 2^-24 at K = 1200.)"""
+    return (1 + (min(k, 64 if dtype == np.float32 else 160) / 6) ** 0.5) * np.finfo(dtype).eps / 2
+
+
 # (no tile, one tile, one row or column more or less than whole tiles of 16, 32 and
 # 48; K of one chunk of 16 and one more or less than whole chunks of 4 and 8 waves,
 # of a run and of slices)
@@ -44,7 +54,7 @@ SHAPES = [(1, 1, 16), (15, 17, 17), (16, 16, 31), (17, 33, 63), (31, 47, 64), (3
 @pytest.mark.parametrize("m,n,k", SHAPES)
 def test_against_higher_precision(env, dtype, m, n, k):
     """A sum of K products in any order is within K roundings of |a| |b|: K / 2 of
-    its last place to nearest."""
+    its last place to nearest; the error's 2-norm within _norm_room."""
     hip, gemm = env
     rng = np.random.default_rng(m + 10 * n + 100 * k)
     a, b = rng.standard_normal((m, k)).astype(dtype), rng.standard_normal((k, n)).astype(dtype)
@@ -52,6 +62,7 @@ def test_against_higher_precision(env, dtype, m, n, k):
     high = np.float64 if dtype == np.float32 else np.longdouble
     product = a.astype(high) @ b.astype(high)
     bound = (k + 4) * np.finfo(dtype).eps / 2 * (np.abs(a).astype(high) @ np.abs(b).astype(high))
+    norm_room = _norm_room(dtype, k) * np.sqrt((product ** 2).sum())
     for ta in (False, True):
         for tb in (False, True):
             for off in (False, True):
@@ -60,6 +71,7 @@ def test_against_higher_precision(env, dtype, m, n, k):
                 gemm(d_a, d_b, d_c, 1.0, 0.0)
                 got = d_c.asnumpy()
                 assert (np.abs(got - product) <= bound).all(), (ta, tb, off)
+                assert np.sqrt(((got - product) ** 2).sum()) <= norm_room, (ta, tb, off)
                 gemm(d_a, d_b, d_c, 1.0, 0.0)
                 assert np.array_equal(d_c.asnumpy(), got)
     wide = rng.standard_normal((m, n + 2)).astype(dtype)
@@ -88,6 +100,7 @@ def test_many_slices_of_a_long_k(env, dtype, m, n, k):
     high = np.float64 if dtype == np.float32 else np.longdouble
     product = a.astype(high) @ b.astype(high)
     bound = (k + 4) * np.finfo(dtype).eps / 2 * (np.abs(a).astype(high) @ np.abs(b).astype(high))
+    norm_room = _norm_room(dtype, k) * np.sqrt((product ** 2).sum())
     wide = rng.standard_normal((m, n + 2)).astype(dtype)
     for ta in (False, True):
         for tb in (False, True):
@@ -99,6 +112,7 @@ def test_many_slices_of_a_long_k(env, dtype, m, n, k):
                 outs.append(d_c.asnumpy())
             assert np.array_equal(outs[0], outs[1])
             assert (np.abs(outs[0] - product) <= bound).all(), (ta, tb)
+            assert np.sqrt(((outs[0] - product) ** 2).sum()) <= norm_room, (ta, tb)
     d_w = hip.asarray(wide)
     gemm(d_a, d_b, d_w[:, 1:n + 1], 1.5, -0.5)
     got = d_w.asnumpy()
