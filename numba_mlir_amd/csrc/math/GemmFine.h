@@ -9,18 +9,19 @@
 //
 // What bounds it: for a result of a few tiles the chunks of K that a wave loads
 // one after the other (0.2 to 0.4 us each); for more, the operands' way into the
-// registers: tiles this small read them from L2 at 10 TB/s and more, and a load of
-// four neighbours of K from each of 16 rows takes the vector cache four times as
-// long as one of whole lines.  (Through LDS, coalesced: float32 2048^3 187 -> 147
-// us, which the bf16 parts do in 105, but float64 1000 x 1100 x 1200 46.6 -> 49
-// and 822 x 641 x 1048 22.5 -> 25.7, one block a CU.)  48 x 48 is the largest
-// tile of float64 that leaves two waves a SIMD.
+// registers: tiles this small read them again and again from L2 (float64 1000 x 1100 x
+// 1200 445 MB in 54 us, 8.3 TB/s), and a load of four neighbours of K from each of 16
+// rows takes the vector cache four times as long as one of whole lines.  (Through LDS,
+// coalesced: float32 2048^3 a fifth faster, which the bf16 parts do in 105 us, but float64
+// 1000 x 1100 x 1200 5 % and 822 x 641 x 1048 14 % slower, one block a CU.)  48 x 48 is
+// the largest tile of float64 that leaves two waves a SIMD.
 //
-// Kernels before (copies, tiles or the strided kernel, folds) / now, us: float32
-// 126 x 1 x 100 11.3 / 3.2, 435 x 73 x 175 17.5 / 3.2, 111 x 290 x 1694 199 / 7.1, 496
-// x 691 x 74 13.2 / 4.7, 83 x 3325 x 852 28.5 / 14.4; float64 75 x 72 x 528 43.4 / 6.6,
-// 583 x 175 x 280 32.9 / 5.7, 2391 x 420 x 140 27.2 / 13.0, 822 x 641 x 1048 55.5 / 25,
-// 4023 x 93 x 2646 94 / 40, 1000 x 1100 x 1200 68.8 / 49.5 (53 TFLOP/s).
+// Kernels before (copies, tiles or the strided kernel, folds) / now, us, medians of 40
+// calls on row-major operands: float32 126 x 1 x 100 11.4 / 3.4, 435 x 73 x 175 17.6 / 3.8,
+// 111 x 290 x 1694 135 / 7.4, 496 x 691 x 74 13.4 / 5.4, 83 x 3325 x 852 28.0 / 21.9; float64
+// 75 x 72 x 528 44.5 / 6.1, 583 x 175 x 280 25.9 / 6.4, 2391 x 420 x 140 25.5 / 13.6, 822 x
+// 641 x 1048 57.3 / 28.8, 4023 x 93 x 2646 70.5 / 45.4, 1000 x 1100 x 1200 71.3 / 56.2 (47
+// TFLOP/s; 53.6 where only this product runs).
 #pragma once
 
 #include <hip/hip_runtime.h>

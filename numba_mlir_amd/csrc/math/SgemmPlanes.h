@@ -10,11 +10,11 @@
 // element instead of 8, laid out as the matrix instructions read it, so that the
 // product kernel moves it to LDS without passing a register and multiplies, 894
 // cycles a slab of 16 of a tile where its matrix instructions take 768.  What
-// bounds it then is the power limit: 1.65 to 1.7 GHz with all CUs at it, 2.4 with
-// four (0.53 and 0.37 us a slab).
+// bounds it then is the power limit: a slab takes 0.53 us with all CUs at it, 0.37 with
+// four, 1.7 and 2.4 GHz.
 //
 // Kernels of a call, us, copies + tiles + fold before / split + tiles + fold now:
-// 2047 x 2049 x 2051 14 + 109 + 15 / 18.5 + 95 + 7.5; calls 877 x 4531 x 1863 130 /
+// 2047 x 2049 x 2051 13.9 + 105.4 + 14.3 / 19.6 + 95.4 + 9.2; calls 877 x 4531 x 1863 130 /
 // 114, 4026 x 1410 x 3158 270 / 237, 5657 x 2051 x 481 130 / 98.  On the way: one
 // wave a SIMD with its loads and LDS reads ahead of the matrix instructions instead
 // of between them 1217 cycles a slab; two blocks a CU 567 us at 4096^3 and twice the
